@@ -9,10 +9,13 @@
 //   gemm_mfma_nt   bf16, A K-contiguous and B K-contiguous (sbk == 1; B = W.t() of a [N, K] weight) or, BNM,
 //                  N-contiguous (sbn == 1; a row-major [K, N] B): 32x32x16 bf16 MFMA, register + LDS staged
 //                  pipeline, GROUP_M-swizzled, XCD-aware tile order.
+//   gemm_stream_nt bf16, K-contiguous A and B, when there are more tiles than one round on the CUs: persistent blocks,
+//                  memory -> LDS loads, 16x16x32 MFMA; the same bits.
 //   gemm_skinny    bf16 with M <= 32, same layout: 16 columns per block, K split over 8 waves, 16x16x32 MFMA.
 //   gemm_mfma_f32  fp32, A K-contiguous, B K- or N-contiguous: 32x32x2 fp32 MFMA (exact products, fp32 sums).
 //   gemm_generic   any dtype/strides/precision: 64x64 tile, 4x4 outputs per thread, fp32 FMA.
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 
@@ -404,6 +407,253 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_nt(const Mfm
       for (int e = 0; e < 8 && n + e < g.N; ++e) d[e] = uint16_t(v[e / 2] >> (16 * (e & 1)));
     }
   }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// bf16 MFMA kernel for many tiles (prompt batches, the LM head of a large batch): the layouts of gemm_mfma_nt with
+// K % 64 == 0 and 16-byte aligned output rows, the same products summed in the same order (its outputs are bitwise
+// gemm_mfma_nt's: a 16x16x32 MFMA adds its 32 products as two 32x32x16 MFMAs do), with or without SILU.
+//
+// What bounds it: at 256x256 tiles the matrix cores want 64 KB of operands per 64-deep k-tile and CU from the L2,
+// twice that or more in LDS fragment reads, and the shader clock falls under the load. Staged through registers
+// (gemm_mfma_nt), the LDS writes and the waits on loads that must return to a register before they can be stored cost
+// the most; here
+//   - the loads go from memory straight into LDS (buffer_load_dwordx4 ... lds: no register, no LDS store
+//     instruction), 1 KB per wave instruction = 8 rows of 64 k; the 16-byte chunk c of a row lies at chunk
+//     c ^ ((row >> 1) & 7), which the lane's global address provides (a DMA load writes LDS linearly);
+//   - NSA / NSB LDS stages per operand. A stage is refilled as soon as the block's waves have read it (one barrier
+//     per k-tile, after the first row of MFMAs of its last k step), its loads spread over SPREAD of the k-tile's
+//     MFMAs: issued back to back they fill the memory pipeline's queue and hold up the MFMAs behind them (8192^3:
+//     824 us in one k step, 815 spread);
+//   - 16x16x32 MFMAs instead of 32x32x16: the same LDS bytes and cycles, 7 % faster (8192^3 815 -> 758 us);
+//   - the blocks are persistent (one per CU) and the k-tiles of a block's tiles are one stream: the next tile's first
+//     k-tiles are in flight during a tile's epilogue, and the epilogue stores straight from registers.
+// The A fragments are single buffered (an A fragment is re-read once its row of MFMAs has been issued), the B
+// fragments double buffered.
+// Measured against gemm_mfma_nt in one process each: 16384 x 6144 x 1024 + SiLU 233.7 -> 203.2 us, 16384 x 1024 x
+// 3072 92.6 -> 84.2, 4099 x 4096 x 1024 47.9 -> 41.7, 4099 x 1024 x 3072 45.9 -> 32.4, 250 x 151936 x 1024 118.8 ->
+// 101.0, 8192^3 886 -> 788 us. With the DMA loads left out 8192^3 takes 674 us, with every load an L2 hit 768 us.
+//
+// Tile order: XCD x takes an eighth of the tiles, in the order of the GROUP_M swizzle, so that its blocks share their
+// operand rows in its L2.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+constexpr int kStreamBlocks = 256;  // one persistent block per CU
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NSA, int NSB, bool SILU>
+__global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_stream_nt(const MfmaArgs g) {
+  constexpr int NW = WAVES_M * WAVES_N, WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 16, FN = WN / 16;
+  constexpr int BK = kBK, KS = BK / 32, NM = FM * FN;    // k steps of 32 and MFMAs per k step
+  constexpr int RPD = 8;                                 // rows per DMA load
+  constexpr int SA = BM * BK * 2, SB = BN * BK * 2;      // bytes of a stage
+  constexpr int DA = BM / RPD / NW, DB = BN / RPD / NW;  // DMA loads per wave and k-tile
+  constexpr int ND = DA + DB, NS = NSA > NSB ? NSA : NSB;
+  static_assert(DA * RPD * NW == BM && DB * RPD * NW == BN, "whole DMA loads per wave");
+  static_assert(FM % 2 == 0 && (!SILU || FN % 2 == 0) && NSA >= 2 && NSB >= 2, "tile shape");
+  static_assert(NSA * SA + NSB * SB <= 160 * 1024, "LDS");
+  // The loads of one refill go out A first when A has no more stages than B, else B first: what is needed sooner.
+  // With `late` = the operand with more stages, the refills issued before the barrier of k-tile t cover k-tile t + 1
+  // but for the youngest late ones: WAIT loads may still be in flight there.
+  constexpr int WAIT = NSA > NSB   ? DA + (NSB - 2) * ND
+                       : NSA < NSB ? DB + (NSA - 2) * ND
+                                   : (NSA - 2) * ND;
+  constexpr int SPREAD = KS * NM - NM / 4;  // MFMAs over which a refill is spread, from the barrier on
+  constexpr int LAST = NM - FN + 1;         // MFMAs from the barrier to the end of the k-tile
+  constexpr int NLAST = SPREAD <= LAST ? ND : (LAST * ND + SPREAD - 1) / SPREAD;  // loads of a refill issued there
+  __shared__ __attribute__((aligned(1024))) char lds[NSA * SA + NSB * SB];
+  const uint32_t lbase = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / 64);
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int num_m = (g.M + BM - 1) / BM, num_n = (g.N + BN - 1) / BN, total = num_m * num_n, nk = g.K / BK;
+  constexpr int kPerXcd = kStreamBlocks / 8;
+  const int xcd = blockIdx.x % 8, tend = int(int64_t(total) * (xcd + 1) / 8);
+  int tile = int(int64_t(total) * xcd / 8) + int(blockIdx.x) / 8;  // then every kPerXcd-th tile below tend
+  if (tile >= tend) return;
+  auto coords = [&](int t, int& m0, int& n0) {
+    const int in_group = kGroupM * num_n, first_m = t / in_group * kGroupM, rows = min(num_m - first_m, kGroupM);
+    m0 = (first_m + t % in_group % rows) * BM;
+    n0 = t % in_group / rows * BN;
+  };
+
+  // Load cursors, one per operand: the k-tile being loaded, its stage, and this lane's byte offsets from the tile's
+  // first row. DMA load i of wave w brings rows 8 (w + NW i) .. +8; rows past M / N repeat the last one. SILU: of each
+  // wave's column tiles the first half are gate rows, the second half the matching up rows.
+  struct Cursor {
+    int tile, kt, stage;
+  };
+  Cursor ca{tile, 0, 0}, cb{tile, 0, 0};
+  uint32_t va[DA], vb[DB];
+  u32x4 ra, rb;  // buffer descriptors
+  auto descriptor = [](const uint16_t* p) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return u32x4{uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(a))),
+                 uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(a >> 32) & 0xffffu)), 0x7fffffffu, 0x00020000u};
+  };
+  const int lrow = wave * RPD + lane / 8;
+  auto locate_a = [&]() {
+    int m0, n0;
+    coords(ca.tile, m0, n0);
+    ra = descriptor(g.a + int64_t(m0) * g.sam);
+#pragma unroll
+    for (int i = 0; i < DA; ++i) {
+      const int row = lrow + i * NW * RPD;
+      va[i] = uint32_t(min(row, g.M - 1 - m0)) * uint32_t(g.sam * 2) + ((lane % 8) ^ ((row >> 1) & 7)) * 16;
+    }
+  };
+  auto locate_b = [&]() {
+    int m0, n0;
+    coords(cb.tile, m0, n0);
+    rb = descriptor(g.w + int64_t(SILU ? n0 / 2 : n0) * g.swn);
+#pragma unroll
+    for (int i = 0; i < DB; ++i) {
+      const int row = lrow + i * NW * RPD;
+      uint32_t r;
+      if constexpr (SILU) {
+        const int n2 = g.N / 2, f = row / 16 % FN;
+        r = uint32_t(min(row / WN * (WN / 2) + f % (FN / 2) * 16 + row % 16, n2 - 1 - n0 / 2)) +
+            (f >= FN / 2 ? uint32_t(n2) : 0u);
+      } else {
+        r = uint32_t(min(row, g.N - 1 - n0));
+      }
+      vb[i] = r * uint32_t(g.swn * 2) + ((lane % 8) ^ ((row >> 1) & 7)) * 16;
+    }
+  };
+  // No output register: the load's only result is 16 bytes per lane at LDS address dst + 16 lane, which the waits
+  // before the barriers below cover.
+  auto dma = [&](const u32x4& rsrc, uint32_t vofs, uint32_t dst, int kt) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(vofs),
+                 "s"(rsrc), "s"(uint32_t(kt) * (BK * 2))
+                 : "memory");
+  };
+  auto dma_q = [&](auto qc) {  // load q of a refill
+    constexpr int q = decltype(qc)::value;
+    constexpr bool is_a = NSA <= NSB ? q < DA : q >= DB;
+    constexpr int i = is_a ? (NSA <= NSB ? q : q - DB) : (NSA <= NSB ? q - DA : q);
+    if constexpr (is_a) dma(ra, va[i], lbase + ca.stage * SA + (wave + NW * i) * 1024, ca.kt);
+    else dma(rb, vb[i], lbase + NSA * SA + cb.stage * SB + (wave + NW * i) * 1024, cb.kt);
+  };
+  // Past the block's last k-tile that one is loaded again, unused, so that the loop has no branch on it.
+  auto next = [&](Cursor& c, int stages) {  // true: another tile
+    c.stage = c.stage + 1 == stages ? 0 : c.stage + 1;
+    if (++c.kt < nk) return false;
+    if (c.tile + kPerXcd >= tend) {
+      c.kt = nk - 1;
+      return false;
+    }
+    c.kt = 0;
+    c.tile += kPerXcd;
+    return true;
+  };
+  locate_a();
+  locate_b();
+  static_for<NS>([&](auto sc) {  // refills -NS .. -1: k-tiles r + NSA of A and r + NSB of B, the last one in part
+    constexpr int r = decltype(sc)::value - NS;
+    if constexpr (r + NSA > 0)
+      if (next(ca, NSA)) locate_a();
+    if constexpr (r + NSB > 0)
+      if (next(cb, NSB)) locate_b();
+    static_for<(r == -1 ? NLAST : ND)>([&](auto qc) {
+      constexpr bool is_a = NSA <= NSB ? decltype(qc)::value < DA : decltype(qc)::value >= DB;
+      if constexpr (r + (is_a ? NSA : NSB) >= 0) dma_q(qc);
+    });
+  });
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WAIT + NLAST) : "memory");
+
+  // Fragments (lane l: row l % 16, k = 8 (l / 16) .. +8 of the k step)
+  bf16x8_t af[FM], bfr[2][FN];
+  const int fr = lane % 16, fq = lane / 16, swz = (fr >> 1) & 7;
+  auto chunk = [&](int kk) { return ((4 * kk + fq) ^ swz) * 16; };
+  auto read_a = [&](int stage, int kk, int i) {
+    af[i] = *reinterpret_cast<const bf16x8_t*>(lds + stage * SA + (wm * WM + i * 16 + fr) * (BK * 2) + chunk(kk));
+  };
+  auto read_b = [&](int stage, int kk, int buf, int j) {
+    bfr[buf][j] = *reinterpret_cast<const bf16x8_t*>(lds + NSA * SA + stage * SB +
+                                                     (wn * WN + j * 16 + fr) * (BK * 2) + chunk(kk));
+  };
+#pragma unroll
+  for (int j = 0; j < FN; ++j) read_b(0, 0, 0, j);
+#pragma unroll
+  for (int i = 0; i < FM; ++i) read_a(0, 0, i);
+  int sa = 0, sb = 0;
+  for (;;) {
+    f32x4_t acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{};
+    for (int kt = 0; kt < nk; ++kt) {
+      const int na = sa + 1 == NSA ? 0 : sa + 1, nb = sb + 1 == NSB ? 0 : sb + 1;
+      static_for<KS * NM>([&](auto xc) {
+        constexpr int kk = decltype(xc)::value / NM, x = decltype(xc)::value % NM, i = x / FN, j = x % FN;
+        constexpr bool last = kk + 1 == KS;
+        // operands swapped: lane l holds row l % 16, columns 4 (l / 16) .. +4 of output tile (i, j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[kk & 1][j], af[i], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (last && x == FN - 1) {
+          // every wave has its fragments of this k-tile and its part of the next one: the stages of this one are free
+          if (next(ca, NSA)) locate_a();
+          if (next(cb, NSB)) locate_b();
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WAIT) : "memory");
+        }
+        constexpr int x0 = last ? FN - 1 : 0;  // the next k step's fragments, from here on
+        if constexpr (x >= x0) {
+          constexpr int step = (NM - 2 * FN) / 2 / FN > 0 ? (NM - 2 * FN) / 2 / FN : 1;
+          if constexpr ((x - x0) % step == 0 && (x - x0) / step < FN)
+            read_b(last ? nb : sb, last ? 0 : kk + 1, (kk + 1) & 1, (x - x0) / step);
+          if constexpr (j == FN - 1) read_a(last ? na : sa, last ? 0 : kk + 1, i);
+        }
+        constexpr int pos = last ? x - (FN - 1) : (kk + 1) * NM + x - (FN - 1);  // MFMAs since the barrier
+        if constexpr (pos >= 0 && pos < SPREAD)
+          static_for<ND>([&](auto qc) {
+            if constexpr (decltype(qc)::value * SPREAD / ND == pos) dma_q(qc);
+          });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      sa = na, sb = nb;
+    }
+    // Epilogue from registers, two 16-row tiles at a time: a lane swap (v_permlane16_swap) gives lane l the 8 columns
+    // 8 (l / 32) .. +8 of row l % 16 of tile i + (l / 16) % 2, one 16-byte store.
+    int m0, n0;
+    coords(tile, m0, n0);
+    constexpr int OC = SILU ? WN / 2 : WN;  // output columns of the wave
+    const int nout = SILU ? g.N / 2 : g.N, nb0 = (SILU ? n0 / 2 : n0) + wn * OC + 8 * (fq >> 1);
+#pragma unroll
+    for (int i = 0; i < FM; i += 2) {
+      const int m = m0 + wm * WM + (i + (fq & 1)) * 16 + fr;
+      uint16_t* crow = g.c + int64_t(m) * g.scm;
+#pragma unroll
+      for (int j = 0; j < OC / 16; ++j) {
+        uint32_t w[2][2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (SILU)
+              v[e] = silu_bf16(round_bf16(acc[i + t][j][e])) * round_bf16(acc[i + t][j + FN / 2][e]);
+            else
+              v[e] = acc[i + t][j][e];
+          }
+          w[t][0] = pack_bf16x2(v[0], v[1]);
+          w[t][1] = pack_bf16x2(v[2], v[3]);
+        }
+        const auto lo = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+        const int n = nb0 + j * 16;
+        if (m < g.M && n < nout) *reinterpret_cast<u32x4*>(crow + n) = u32x4{lo[0], hi[0], lo[1], hi[1]};
+      }
+    }
+    tile += kPerXcd;
+    if (tile >= tend) break;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may land in LDS that the block has given away
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -1260,6 +1510,52 @@ int launch_mfma_shape(const MfmaArgs& g, hipStream_t s) {
   }
 }
 
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NSA, int NSB, bool SILU>
+int launch_stream(const MfmaArgs& g, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_stream_nt<BM, BN, WAVES_M, WAVES_N, NSA, NSB, SILU>), dim3(kStreamBlocks),
+                     dim3(WAVES_M * WAVES_N * 64), 0, s, g);
+  return check_launch("matmul");
+}
+
+// Whether gemm_stream_nt takes the product: K in whole k-tiles, output rows in whole 16-byte pieces, and a tile's
+// operand rows within the 2 GiB that a buffer load's offset reaches (with SILU from a gate row to its up row).
+template <bool SILU>
+bool stream_layout(const MfmaArgs& g) {
+  const int64_t nout = SILU ? g.N / 2 : g.N, reach = int64_t(1) << 30;  // elements
+  const int64_t tiles = int64_t((g.M + 127) / 128) * ((g.N + 127) / 128);
+  return g.K % kBK == 0 && nout % 8 == 0 && g.scm % 8 == 0 && aligned16(g.c) && tiles < (int64_t(1) << 30) &&
+         256 * g.sam + g.K < reach && (256 + (SILU ? nout : 0)) * g.swn + g.K < reach;
+}
+
+// gemm_stream_nt's tile shape: rounds of one tile per CU, each nk * per_ktile + fixed us (its last round, run by fewer
+// blocks at a higher clock, counts half and half by how full it is), fitted on MI355X to the seven shapes at M = 512
+// .. 16384 x six (N, K) of hidden 1024 and 2048 and to the LM head of 250 rows; the model's pick was within 2 % of the
+// best of the seven at all but one of the 45 launches that it decides.
+template <bool SILU>
+int launch_stream_shape(const MfmaArgs& g, hipStream_t s) {
+  struct Shape { int bm, bn; double per_ktile, fixed; };
+  constexpr Shape shapes[] = {{256, 256, 1.60, 7.0}, {256, 192, 1.22, 5.5}, {192, 256, 1.23, 5.5}, {256, 128, 0.87, 3.8},
+                              {128, 256, 0.84, 4.2}, {128, 192, 0.645, 3.4}, {192, 128, 0.715, 4.1}};
+  int best = 0;
+  double best_cost = 0.0;
+  for (int i = 0; i < 7; ++i) {
+    const int64_t tiles = int64_t((g.M + shapes[i].bm - 1) / shapes[i].bm) * ((g.N + shapes[i].bn - 1) / shapes[i].bn);
+    const int64_t full = tiles / kStreamBlocks, rem = tiles % kStreamBlocks;
+    const double rounds = double(full) + (rem ? 0.5 + 0.5 * double(rem) / kStreamBlocks : 0.0);
+    const double cost = rounds * (g.K / kBK * shapes[i].per_ktile + shapes[i].fixed);
+    if (i == 0 || cost < best_cost) best = i, best_cost = cost;
+  }
+  switch (best) {
+    case 0: return launch_stream<256, 256, 2, 4, 2, 3, SILU>(g, s);
+    case 1: return launch_stream<256, 192, 4, 2, 2, 3, SILU>(g, s);
+    case 2: return launch_stream<192, 256, 2, 4, 3, 2, SILU>(g, s);
+    case 3: return launch_stream<256, 128, 4, 2, 3, 3, SILU>(g, s);
+    case 4: return launch_stream<128, 256, 2, 4, 3, 3, SILU>(g, s);
+    case 5: return launch_stream<128, 192, 4, 2, 4, 4, SILU>(g, s);
+    default: return launch_stream<192, 128, 2, 4, 4, 4, SILU>(g, s);
+  }
+}
+
 // N-contiguous B: the tile kernel at every M (the skinny kernels read K-contiguous W rows straight into MFMA
 // operands).
 int launch_mfma_bnm(const MfmaArgs& g, hipStream_t s) {
@@ -1395,6 +1691,14 @@ int launch_mfma_auto(const MfmaArgs& g, hipStream_t s) {
     return check_launch("matmul");
   }
   if (g.M <= 64 && g.K >= 2048) return launch_skinny<2, SILU>(g, s);  // wider outputs: the M <= 32 tilings
+  // More tiles than one round of 128x128 (or 64x128) ones: the streaming kernel. Within one round gemm_mfma_nt's small
+  // tiles, with their operands in flight in registers, are as fast or faster (1024 x 4096 x 1024 12.8 us against 14.0,
+  // 2048 x 1024 x 3072 18.7 against 19.5; 1536 x 4096 x 1024 takes 20.0 against 18.5 here), and for up to 128 rows of
+  // the LM head too (100 x 151936 x 1024 73.3 us against 74.6).
+  const int64_t n128 = (g.N + 127) / 128;
+  if (g.M > 128 && int64_t((g.M + 127) / 128) * n128 > kStreamBlocks &&
+      stream_layout<SILU>(g))
+    return launch_stream_shape<SILU>(g, s);
   const int nk = (g.K + kBK - 1) / kBK;
   if (g.K % kBK != 0) return launch_mfma_shape<1, true, SILU>(g, s);
   if (nk % 2 == 0) return launch_mfma_shape<2, false, SILU>(g, s);

@@ -17,7 +17,7 @@ import pytest
 import torch
 
 import oracle
-from nanovllm_hip.kernels import matmul
+from nanovllm_hip.kernels import matmul, matmul_silu_and_mul, silu_and_mul
 
 pytestmark = pytest.mark.gpu
 
@@ -264,3 +264,34 @@ def test_matmul_silu_mul_is_bitwise_the_two_step_result(M, I, K):
     # and against the oracle composition (float64 product rounded to bf16, then the reference's silu * up)
     ref = oracle.silu_and_mul(oracle.matmul_fp64(x.cpu(), w.cpu().t()).to(torch.bfloat16))
     torch.testing.assert_close(fused.cpu().float(), ref.float(), rtol=1.6e-2, atol=2e-2)
+
+
+# More tiles than one round of 128x128: gemm_stream_nt in each of its seven tile shapes (256x256, 192x256, 128x256,
+# 256x128, 128x192, 256x192, 192x128, in the order of their first rows below), one to 16 k-tiles per tile, the last
+# tiles of rows and columns cut short.
+STREAM_SHAPES = [(1025, 10760, 64), (777, 9224, 128), (777, 6920, 320), (643, 8288, 192), (257, 10888, 64),
+                 (641, 11112, 128), (543, 10128, 320), (1025, 10760, 1024), (257, 10888, 1024), (4099, 1352, 1024)]
+
+
+@pytest.mark.parametrize("M,N,K", STREAM_SHAPES)
+def test_many_tiles_are_bitwise_the_staged_kernel(M, N, K):
+    """The N-contiguous layout of the same B runs gemm_mfma_nt, whose k order the streaming kernel keeps: the two
+    products are bitwise equal, also from strided rows of A and W, and within the bf16 tolerance of fp64."""
+    g = torch.Generator("cpu").manual_seed(M + N + K)
+    a = (torch.randn(M, K + 24, generator=g) / math.sqrt(K)).to(torch.bfloat16).to(DEV)[:, :K]
+    w = torch.randn(N, K + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :K]
+    c = matmul(a, w.t())
+    assert torch.equal(c, matmul(a, w.t().contiguous()))
+    assert torch.equal(c, matmul(a.contiguous(), w.contiguous().t()))
+    rows = torch.tensor([0, 1, M // 2, M - 2, M - 1])
+    ref = oracle.matmul_fp64(a.cpu()[rows], w.cpu().t())
+    torch.testing.assert_close(c.cpu()[rows].double(), ref, rtol=1.6e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("M,N,K", STREAM_SHAPES)
+def test_many_tiles_silu_is_bitwise_two_step(M, N, K):
+    inter = (N // 2 + 7) // 8 * 8
+    g = torch.Generator("cpu").manual_seed(M + N + K)
+    a = (torch.randn(M, K, generator=g) / math.sqrt(K)).to(torch.bfloat16).to(DEV)
+    w = torch.randn(2 * inter, K, generator=g).to(torch.bfloat16).to(DEV)
+    assert torch.equal(matmul_silu_and_mul(a, w), silu_and_mul(matmul(a, w.t())))
