@@ -10,6 +10,7 @@ import os
 import torch  # noqa: F401  (must be loaded before the HIP library, see above)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libnvhip.so")
+TORCH_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libnvhip_torch.so")  # the torch ops
 ABI_VERSION = 7
 
 NVHIP_OK = 0

@@ -45,6 +45,12 @@ def flash_attn_with_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
 paged_decode_attention = flash_attn_with_kvcache
 
 
+def _packed_heads(t, D):
+    st = t.stride()
+    return (st[2] == 1 and st[1] == D and st[0] % 8 == 0 and t.dtype == torch.bfloat16
+            and t.data_ptr() % 16 == 0)
+
+
 def qk_norm_rope_kv_decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, positions: torch.Tensor,
                                      q_weight: torch.Tensor, k_weight: torch.Tensor, eps: float,
                                      cos_sin_cache: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -66,8 +72,7 @@ def qk_norm_rope_kv_decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.
     assert k_cache.dim() == 4 and k_cache.shape == v_cache.shape and k_cache.shape[3] == D
     assert k_cache.dtype == v_cache.dtype == torch.bfloat16
     ok = (D in (64, 128) and Hq % Hkv == 0 and Hq // Hkv <= 16 and k.shape == v.shape == (B, Hkv, D)
-          and all(t.dtype == torch.bfloat16 and t.stride(2) == 1 and t.stride(1) == D and t.stride(0) % 8 == 0
-                  and t.data_ptr() % 16 == 0 for t in (q, k, v))
+          and _packed_heads(q, D) and _packed_heads(k, D) and _packed_heads(v, D)
           and q_weight.is_contiguous() and k_weight.is_contiguous() and q_weight.data_ptr() % 16 == 0
           and k_weight.data_ptr() % 16 == 0 and cs.dtype == torch.float32 and cs.stride(1) == 1
           and cs.shape[1] == D and cs.stride(0) % 4 == 0 and cs.data_ptr() % 16 == 0

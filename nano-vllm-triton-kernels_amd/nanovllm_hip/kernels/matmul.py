@@ -32,12 +32,16 @@ def matmul_silu_and_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.
     return torch.ops.nvhip.matmul_silu_mul(x, gate_up_weight)
 
 
+def _rows16(t):
+    """Unit element stride and 16-byte aligned rows (of a vector: an aligned start)."""
+    st = t.stride()
+    return st[-1] == 1 and t.data_ptr() % 16 == 0 and (len(st) != 2 or st[0] % 8 == 0)
+
+
 def _fusable(x, residual, norm_w, weight):
     M, K = x.shape
-    tensors = [x, norm_w, weight] + ([residual] if residual is not None else [])
     return (1 <= M <= 32 and K in (1024, 2048) and x.dtype == norm_w.dtype == weight.dtype == torch.bfloat16
-            and all(t.stride(-1) == 1 and t.data_ptr() % 16 == 0 for t in tensors)
-            and all(t.stride(0) % 8 == 0 for t in tensors if t.dim() == 2))
+            and _rows16(x) and _rows16(norm_w) and _rows16(weight) and (residual is None or _rows16(residual)))
 
 
 def rms_norm_matmul(x: torch.Tensor, norm_w: torch.Tensor, eps: float, weight: torch.Tensor,

@@ -112,3 +112,11 @@ def test_model_latches_the_kernel_backend_at_construction():
             Qwen3(cfg, "meta")
     finally:
         kernels.backend = old
+
+
+def test_every_op_has_its_native_implementation():
+    from nanovllm_hip import ops
+    defined = {s.name for s in torch._C._jit_get_all_schemas() if s.name.startswith("nvhip::")}
+    assert defined == {f"nvhip::{name}" for name in ops._OPS}
+    for name in ops._OPS:
+        assert torch._C._dispatch_has_kernel_for_dispatch_key(f"nvhip::{name}", "CUDA"), name
