@@ -295,3 +295,63 @@ def test_many_tiles_silu_is_bitwise_two_step(M, N, K):
     a = (torch.randn(M, K, generator=g) / math.sqrt(K)).to(torch.bfloat16).to(DEV)
     w = torch.randn(2 * inter, K, generator=g).to(torch.bfloat16).to(DEV)
     assert torch.equal(matmul_silu_and_mul(a, w), silu_and_mul(matmul(a, w.t())))
+
+
+# One shape per tile of gemm_split_f32 (64x64, 128x128, 256x128), cut short in rows, columns and k.
+F32_SHAPES = [(301, 200, 100), (2044, 2044, 36), (2044, 4092, 44), (67, 68, 4)]
+
+
+def _f32_operands(M, N, K, nmajor, seed, a_scale=1.0, b_scale=1.0):
+    g = torch.Generator("cpu").manual_seed(seed)
+    a = (torch.randn(M, K, generator=g) * a_scale).to(DEV)
+    b = (torch.randn(K, N, generator=g) * b_scale).to(DEV)
+    return a, b if nmajor else b.t().contiguous().t()
+
+
+def _f64_product(a, b, prec):
+    if prec == "tf32":
+        a, b = (torch.from_numpy(_round_tf32(x.cpu().contiguous().numpy())) for x in (a, b))
+    return a.cpu().double() @ b.cpu().double()
+
+
+def _round_tf32(x):
+    u = x.view(np.uint32)
+    r = ((u + 0xfff + ((u >> 13) & 1)) & ~np.uint32(0x1fff)).view(np.float32)
+    return np.where(np.isfinite(x), r, x).astype(np.float32)
+
+
+@pytest.mark.parametrize("M,N,K", F32_SHAPES)
+@pytest.mark.parametrize("nmajor", [False, True])
+@pytest.mark.parametrize("prec", ["ieee", "tf32"])
+@pytest.mark.parametrize("a_scale,b_scale", [(1.0, 1.0), (2.0 ** -107, 2.0 ** 100), (2.0 ** 60, 2.0 ** 55),
+                                             (2.0 ** -124, 2.0 ** 100)])
+def test_fp32_parts_keep_fp32_accuracy(M, N, K, nmajor, prec, a_scale, b_scale):
+    """The bf16 parts of fp32 (tf32) inputs give the fp32 product: each of K products and sums rounds at 2^-24 of the
+    running sum, which is at most the product's scale sqrt(K), so the 2-norm of the error stays under sqrt(K) 2^-24 of
+    the result's. At 2^-107 the parts end just above the smallest bf16 denormal, at 2^-124 the fp32 MFMAs take over."""
+    a, b = _f32_operands(M, N, K, nmajor, M + K, a_scale, b_scale)
+    ref = _f64_product(a, b, prec)
+    err = (matmul(a, b, prec).cpu().double() - ref).norm() / ref.norm()
+    assert err < math.sqrt(K) * 2.0 ** -24, float(err)
+
+
+@pytest.mark.parametrize("M,N,K", F32_SHAPES)
+@pytest.mark.parametrize("nmajor", [False, True])
+@pytest.mark.parametrize("prec", ["ieee", "tf32"])
+def test_fp32_values_without_parts(M, N, K, nmajor, prec):
+    """Infinities, NaN, the largest finite values and denormals in single rows and columns: those outputs are what fp32
+    arithmetic gives, and the others keep their accuracy."""
+    a, b = _f32_operands(M, N, K, nmajor, M + K, 1.0, 2.0 ** -8)
+    a[3, 1], a[5, 0], a[7, 2], a[9, 3], a[11] = math.inf, -math.inf, math.nan, 3.4e38, 2.0 ** -130
+    b[0, 4], b[1, 6], b[:, 8] = math.inf, 3.3e38, 2.0 ** -140
+    c = matmul(a, b, prec).cpu()
+    ref = _f64_product(a, b, prec)
+    ref32 = ref.float()
+    assert torch.equal(c.isnan(), ref32.isnan())
+    assert torch.equal(c[c.isinf()], ref32[c.isinf()]) and torch.equal(c.isinf(), ref32.isinf())
+    rows = [m for m in range(M) if m not in (3, 5, 7, 9, 11, M - 1)]
+    cols = [n for n in range(N) if n not in (4, 6, 8, N - 1)]
+    got, want = c[rows][:, cols].double(), ref[rows][:, cols]
+    assert (got - want).norm() / want.norm() < math.sqrt(K) * 2.0 ** -24
+    tiny = c[11, cols].double()  # denormal times normal: fp32's own spacing there is 2^-149
+    torch.testing.assert_close(tiny, ref[11, cols], rtol=1e-5, atol=K * 2.0 ** -149)
