@@ -32,6 +32,8 @@
 // each (query tile, sequence, head group) is cut into key ranges run by separate blocks; each writes its queries'
 // (max, sum, O) records and prefill_combine merges them in split order.
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "decode_attention.h"
 
@@ -538,6 +540,400 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
                   pack_bf16x2(o[t][4 * rr + 2] * inv, o[t][4 * rr + 3] * inv)};
 }
 
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// The prefill attention of one sequence over the paged cache (a prompt chunk and its cached prefix), D = 128, with
+// cache blocks of whole key tiles: the grid, the query tiles, the key splits and the arithmetic of
+// prefill_attention_kernel, for a block of 4 waves in which a wave owns 64 queries.
+//
+// What bounded prefill_attention_kernel here: every K and V fragment that a wave of 32 queries reads from LDS feeds one
+// MFMA (128 bytes per clock and CU, the LDS rate), the K / V tiles pass through registers with per-key row arithmetic,
+// and the two waves of a SIMD run the softmax and the matrix products in phase, so they add up (a probe: an MFMA of 32
+// clocks leaves room for 4-5 other instructions of its SIMD, and 64 MFMAs and the ~450 others of a tile have to be
+// mixed to fit). Here
+//   - a fragment read from LDS feeds two MFMAs (64 queries per wave, one wave per SIMD: O and Q in 192 accumulation
+//     registers, two tiles' scores in 128 vector registers);
+//   - K and V tiles go from memory to LDS without registers (global_load_lds, a wave's instruction brings 4 keys), two
+//     tiles ahead; a key tile lies in one cache block, so its address is one scalar table entry. Chunk c of K row r
+//     lies at chunk c ^ (r & 15), of V row r at c ^ 4 (r & 3): fragment and transpose reads hit distinct banks;
+//   - the stream of a tile is mixed by hand: the scores of the next tile between the probabilities of this one, P.V
+//     between the rest of them and the next tile's maxima, one memory load per MFMA behind the barrier.
+// The matrix instructions are inline asm, because the compiler's own choice keeps all results in accumulation registers
+// and moves the scores back and forth. It does not know their timing, so nothing may read a result, or write an operand
+// with a vector instruction, right before or after one: every such pair below lies several MFMAs apart, or behind the
+// s_nop fences.
+// 2048 queries over 14001 cached keys (16 / 8 heads): 326 -> 258-268 us with the q/k norm kernel, 0.77 -> 0.96 PFLOP/s;
+// 256 over 3840 38.5 -> 37. On contiguous keys it was no faster than prefill_attention_kernel (8192 tokens 257-261 us
+// against 266, 16 x 256 tokens 19.5 against 16.6), which keeps those.
+__device__ const uint32_t kZeroRow[64] = {};  // what the keys of an invalid cache block read
+
+constexpr int kWideThreads = 256;
+
+template <int HB>
+__global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const PrefillArgs g) {
+  constexpr int D = 128, kBQ = block_queries(HB), kHeadThreads = kWideThreads / HB;
+  constexpr int NK = 3, NV = 4, TILE = kBK * D * 2;  // LDS slots of K and V tiles, bytes of a tile
+  constexpr int LOADS = 8;                           // memory -> LDS loads per wave and event (4 of K, 4 of V)
+  __shared__ __attribute__((aligned(1024))) char lds[(NK + NV) * TILE];
+  const uint32_t lbase = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
+
+  const int ntile = g.qtiles * g.splits, nblk = int(gridDim.x), ngrp = nblk / ntile;
+  int grp, ci;
+  if (nblk % 8 == 0 && (nblk / 8) % ntile == 0) {
+    const int gx = nblk / 8 / ntile, r = blockIdx.x / 8;
+    grp = (r % gx) * 8 + blockIdx.x % 8;
+    ci = r / gx;
+  } else {
+    grp = blockIdx.x % ngrp;
+    ci = blockIdx.x / ngrp;
+  }
+  const int qt = g.qtiles - 1 - ci / g.splits, split = ci % g.splits;
+  const int b = grp / g.nhg, hg = grp % g.nhg;
+  const int h = hg * HB + int(threadIdx.x) / kHeadThreads, kvh = (hg * HB) / g.G;
+  const int q0s = g.cu_q[b], lq = g.cu_q[b + 1] - q0s;
+  const int lk = g.cu_k[b + 1] - g.cu_k[b];
+  const int k_beg = split * g.split_len;
+  const int k_hi = split == g.splits - 1 ? INT32_MAX : k_beg + g.split_len;
+  const int k_stop = g.causal ? min(min(lk, lk - lq + min(qt * kBQ + kBQ, lq)), k_hi) : min(lk, k_hi);
+  if (qt * kBQ >= lq || k_stop <= k_beg) {
+    const int r = int(threadIdx.x) % kHeadThreads;
+    for (int q = qt * kBQ + r; q < min(qt * kBQ + kBQ, lq); q += kHeadThreads) {
+      const int64_t row = q0s + q;
+      if (g.splits > 1) {
+        if (row >= g.ws_rows) return;
+        const int64_t rec = (int64_t(split) * g.ws_rows + row) * g.Hq + h;
+        float* o = g.ws + rec * D;
+        for (int d = 0; d < D; ++d) o[d] = 0.0f;
+        *reinterpret_cast<f32x2*>(g.ws + int64_t(g.splits) * g.ws_rows * g.Hq * D + 2 * rec) = f32x2{-INFINITY, 0.0f};
+      } else {
+        uint16_t* o = g.out + row * g.o_st + int64_t(h) * g.o_sh;
+        for (int d = 0; d < D; ++d) o[d] = 0;
+      }
+    }
+    return;
+  }
+  const int tid = threadIdx.x, lane = tid % 64, bwave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int wave = __builtin_amdgcn_readfirstlane((tid % kHeadThreads) / 64);
+  const int ql = lane % 32, hf = lane / 32;
+  const int wave_q0 = qt * kBQ + 64 * wave;  // the wave's first query; lane: queries wave_q0 + 32 qh + ql
+
+  bf16x8_t qf[2][8];
+#pragma unroll
+  for (int qh = 0; qh < 2; ++qh) {
+    const int qi = wave_q0 + 32 * qh + ql;
+    const bool ok = qi < lq;
+    const uint16_t* qp = g.q + int64_t(q0s + (ok ? qi : 0)) * g.q_st + int64_t(h) * g.q_sh + 8 * hf;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) qf[qh][c] = ok ? *reinterpret_cast<const bf16x8_t*>(qp + 16 * c) : bf16x8_t{};
+  }
+  const int diag = lk - lq;
+  const int nt = (k_stop - k_beg + kBK - 1) / kBK, last = k_beg + (nt - 1) * kBK;
+
+  // loads
+  const int32_t* bt_row = g.bt + int64_t(b) * g.max_blocks;
+  const uint32_t row_bytes = uint32_t(g.Hkv) * D * 2;
+  uint32_t kofs[4], vofs[4];
+  const int lr = lane / 16, lc = lane % 16;
+  auto offsets = [&](int v_rows, int k_rows) {  // rows of the tiles that exist; past them the last one again
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 4 * (bwave + 4 * j) + lr;
+      kofs[j] = uint32_t(min(row, k_rows - 1)) * row_bytes + ((lc ^ (row & 15)) * 16);
+      vofs[j] = uint32_t(min(row, v_rows - 1)) * row_bytes + ((lc ^ ((row & 3) << 2)) * 16);
+    }
+  };
+  offsets(kBK, kBK);
+  // Where the K tile loaded next lies, and the V tile, which is the K tile of the event before: first key (the last
+  // tile is loaded again past the end), cache block (its table entry fetched an event ahead) and place in it. An invalid
+  // block reads 16-byte pieces of kZeroRow: keys and values of zero.
+  int k_kt = k_beg, v_kt = k_beg, k_to = 0, v_to = NV - 1;  // (the first event's V tile is not loaded)
+  int blk_idx = k_beg / g.bs, blk_ofs = k_beg % g.bs, blk = load_uniform(bt_row + blk_idx);
+  int64_t elem = 0;
+  uint32_t k_mask = 0, v_mask = 0, k_dst = 0, v_dst = 0;
+  uint64_t k_at = 0, v_at = 0;
+  const uint64_t zero_row = reinterpret_cast<uint64_t>(kZeroRow);
+  auto dma = [&](uint32_t dst, uint32_t ofs, uint64_t p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(ofs), "s"(p)
+                 : "memory");
+  };
+  // One event's loads: next_load() prepares them, load(0 .. 3) issues V's and load(4 .. 7) K's.
+  auto next_load = [&]() {
+    v_mask = k_mask;
+    v_at = v_mask == 0xffffffffu ? reinterpret_cast<uint64_t>(g.v + elem) : zero_row;
+    v_dst = lbase + (NK + v_to) * TILE + bwave * 1024;
+    k_mask = blk >= 0 && blk < g.num_blocks ? 0xffffffffu : 0xf0u;
+    elem = ((int64_t(blk) * g.bs + blk_ofs) * g.Hkv + kvh) * D;
+    k_at = k_mask == 0xffffffffu ? reinterpret_cast<uint64_t>(g.k + elem) : zero_row;
+    k_dst = lbase + k_to * TILE + bwave * 1024;
+    if (k_kt + kBK > lk) offsets(min(kBK, lk - v_kt), lk - k_kt);
+    v_to = v_to + 1 == NV ? 0 : v_to + 1;
+    k_to = k_to + 1 == NK ? 0 : k_to + 1;
+    v_kt = k_kt;
+    if (k_kt < last) {
+      k_kt += kBK;
+      blk_ofs += kBK;
+      if (blk_ofs == g.bs) blk_ofs = 0, ++blk_idx;
+      blk = load_uniform(bt_row + blk_idx);
+    }
+  };
+  auto load = [&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    if constexpr (j < 4) dma(v_dst + j * 4096, vofs[j] & v_mask, v_at);
+    else dma(k_dst + (j - 4) * 4096, kofs[j - 4] & k_mask, k_at);
+  };
+  next_load();
+  static_for<4>([&](auto jc) { load(std::integral_constant<int, decltype(jc)::value + 4>{}); });
+  next_load();
+  static_for<8>([&](auto jc) { load(jc); });
+  next_load();
+  static_for<8>([&](auto jc) { load(jc); });
+
+  f32x16_t o[4][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int qh = 0; qh < 2; ++qh) o[t][qh] = f32x16_t{};
+  auto fence_o = [&]() {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) asm volatile("s_nop 15" : "+a"(o[t][0]), "+a"(o[t][1]));
+  };
+  fence_o();
+#pragma unroll
+  for (int qh = 0; qh < 2; ++qh)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) asm volatile("s_nop 1" : "+a"(qf[qh][c]));
+
+  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f}, tmax[2];
+  // fragment addresses
+  const uint32_t ka = uint32_t(ql) * 256, kx = uint32_t(hf ^ (ql & 15)) << 4;
+  const uint32_t va = uint32_t(4 * hf + (lane % 16) / 4) * 256 + (lane % 2) * 8;
+  const uint32_t vx = uint32_t((2 * (ql / 16) + (lane % 4) / 2) ^ (((lane % 16) / 4) << 2)) << 4;
+  auto read_k = [&](int slot, int u, int c) {
+    return *reinterpret_cast<const bf16x8_t*>(lds + slot * TILE + u * 32 * 256 + ka + ((uint32_t(c) << 5) ^ kx));
+  };
+  auto read_v = [&](int slot, int u, int j, int t) {
+    const uint16_t* p = reinterpret_cast<const uint16_t*>(lds + (NK + slot) * TILE + (32 * u + 16 * j) * 256 + va +
+                                                          ((uint32_t(t) << 6) ^ vx));
+    const u32x2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 8 * D);
+    return __builtin_bit_cast(bf16x8_t, u32x4{lo[0], lo[1], hi[0], hi[1]});
+  };
+  using Scores = f32x16_t[2][2];  // [u][qh]
+  auto mask = [&](Scores& s, int kt0) {  // where the tile at kt0 needs it
+    if (kt0 + kBK <= lk && (!g.causal || kt0 + kBK - 1 <= diag + wave_q0)) return;
+#pragma unroll
+    for (int qh = 0; qh < 2; ++qh) {
+      const int lim = min(lk - 1, g.causal ? diag + wave_q0 + 32 * qh + ql : lk - 1) - kt0 - 4 * hf;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (32 * u + 8 * (r / 4) + r % 4 > lim) s[u][qh][r] = -INFINITY;
+    }
+  };
+  auto max_step = [&](const Scores& s, auto kc) {  // step k of 32: two scores of a query half
+    constexpr int k = decltype(kc)::value, qh = k % 2, e = k / 2 * 2;
+    const float m = k < 2 ? -INFINITY : tmax[qh];
+    tmax[qh] = fmaxf(fmaxf(m, s[e / 16][qh][e % 16]), s[e / 16][qh][e % 16 + 1]);
+  };
+  auto max_done = [&]() {
+#pragma unroll
+    for (int qh = 0; qh < 2; ++qh) tmax[qh] = pair32_max(tmax[qh]) * g.scale_log2;
+  };
+  int k_slot = 0, v_slot = 0;  // K tile of the next scores, V tile of the next P.V
+  int kt0 = k_beg;             // tile of the current iteration
+  bf16x8_t kf[4];
+  auto scores_mfma = [&](Scores& s, auto xc) {  // MFMA x: step n = 2 c + u of query half x % 2
+    constexpr int x = decltype(xc)::value, n = x / 2, c = n / 2, u = n % 2, qh = x % 2;
+    if constexpr (c == 0)
+      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s[u][qh]) : "v"(kf[n % 4]), "a"(qf[qh][c]));
+    else
+      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[u][qh]) : "v"(kf[n % 4]), "a"(qf[qh][c]));
+    if constexpr (qh == 1 && n + 4 < 16) kf[n % 4] = read_k(k_slot, (n + 4) % 2, (n + 4) / 2);
+  };
+  auto first_k = [&]() {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) kf[n] = read_k(k_slot, n % 2, n / 2);
+  };
+  auto next_slot = [](int& x, int n) { x = x + 1 == n ? 0 : x + 1; };
+  Scores sa, sb;
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * LOADS) : "memory");
+  first_k();
+  static_for<32>([&](auto xc) { scores_mfma(sa, xc); });
+  next_slot(k_slot, NK);
+  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(sa[0][0]), "+v"(sa[0][1]), "+v"(sa[1][0]), "+v"(sa[1][1]));
+  mask(sa, kt0);
+  static_for<32>([&](auto kc) { max_step(sa, kc); });
+  max_done();
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LOADS) : "memory");
+  first_k();
+  next_load();
+  static_for<8>([&](auto jc) { load(jc); });
+
+  constexpr float kLazy = 8.0f;
+  auto iteration = [&](Scores& s, Scores& sn) {
+    // move the reference maxima of this tile's scores
+    bool move[2];
+#pragma unroll
+    for (int qh = 0; qh < 2; ++qh) move[qh] = tmax[qh] > m_run[qh] + kLazy;
+    if (__ballot(move[0] || move[1]) != 0) {
+      float alpha[2];
+#pragma unroll
+      for (int qh = 0; qh < 2; ++qh) {
+        alpha[qh] = move[qh] ? __builtin_amdgcn_exp2f(m_run[qh] - tmax[qh]) : 1.0f;
+        if (move[qh]) m_run[qh] = tmax[qh];
+        l_run[qh] *= alpha[qh];
+      }
+      if (kt0 != k_beg) {
+        fence_o();
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int qh = 0; qh < 2; ++qh) o[t][qh] *= alpha[qh];
+        fence_o();
+      }
+    }
+    float m_use[2];
+#pragma unroll
+    for (int qh = 0; qh < 2; ++qh) m_use[qh] = m_run[qh] == -INFINITY ? 0.0f : m_run[qh];
+    u32x4 pf[2][2][2];  // [u][j][qh]
+    auto pair = [&](auto yc) {  // probabilities 2 (y % 4), + 1 of group y / 4
+      constexpr int y = decltype(yc)::value, grp8 = y / 4, u = grp8 / 4, j = grp8 / 2 % 2, qh = grp8 % 2, e = y % 4;
+      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][qh][8 * j + 2 * e], g.scale_log2, -m_use[qh]));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][qh][8 * j + 2 * e + 1], g.scale_log2, -m_use[qh]));
+      l_run[qh] += p0;
+      l_run[qh] += p1;
+      uint32_t w = pack_bf16x2(p0, p1);
+      asm volatile("" : "+v"(w), "+v"(l_run[qh]));  // here, not where the sums are wanted (the p would stay live)
+      pf[u][j][qh][e] = w;
+    };
+    bf16x8_t vf[4];
+    // the next tile's scores over three quarters of this tile's probabilities
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<32>([&](auto xc) {
+      constexpr int x = decltype(xc)::value;
+      scores_mfma(sn, xc);
+      static_for<24>([&](auto yc) {
+        if constexpr (decltype(yc)::value * 32 / 24 == x) pair(yc);
+      });
+      if constexpr (x >= 28) vf[x - 28] = read_v(v_slot, 0, 0, x - 28);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    next_slot(k_slot, NK);
+    // P.V: MFMA x: step n = (u, j, t) of query half x % 2
+    static_for<32>([&](auto xc) {
+      constexpr int x = decltype(xc)::value, n = x / 2, u = n / 8, j = n / 4 % 2, t = n % 4, qh = x % 2;
+      if constexpr (x == 16) {
+        // K(next + 1) and V(next) have landed, and everybody has read K(next) and the V before this one: their slots
+        // are free
+        asm volatile("" : "+v"(sn[0][0]), "+v"(sn[0][1]), "+v"(sn[1][0]), "+v"(sn[1][1]));
+        mask(sn, kt0 + kBK);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS) : "memory");
+        next_load();
+      }
+      if constexpr (x >= 16 && x < 24) load(std::integral_constant<int, x - 16>{});
+      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(o[t][qh]) : "v"(vf[n % 4]), "v"(pf[u][j][qh]));
+      if constexpr (qh == 1 && n + 4 < 16) vf[n % 4] = read_v(v_slot, (n + 4) / 8, (n + 4) / 4 % 2, (n + 4) % 4);
+      if constexpr (x < 16 && x % 2 == 0) pair(std::integral_constant<int, 24 + x / 2>{});
+      if constexpr (x >= 17 && x < 31) {
+        static_for<32>([&](auto kc) {
+          if constexpr (decltype(kc)::value * 14 / 32 == x - 17) max_step(sn, kc);
+        });
+        asm volatile("" : "+v"(tmax[0]), "+v"(tmax[1]));
+      }
+      if constexpr (x == 31) max_done();
+      if constexpr (x >= 28) kf[x - 28] = read_k(k_slot, x % 2, (x - 28) / 2);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    next_slot(v_slot, NV);
+    kt0 += kBK;
+  };
+  // two copies, so that a tile's scores stay in the registers that the matrix cores wrote them to; the last iteration
+  // computes scores of a tile loaded again, unused
+  for (int left = nt;;) {
+    iteration(sa, sb);
+    if (--left == 0) break;
+    iteration(sb, sa);
+    if (--left == 0) break;
+  }
+  fence_o();
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the LDS is free
+
+#pragma unroll
+  for (int qh = 0; qh < 2; ++qh) {
+    const int q0 = wave_q0 + 32 * qh, qi_lane = q0 + ql;
+    const float l = pair32_sum(l_run[qh]);
+    if (g.splits > 1) {
+      const int nq = min(32, min(lq, int(min<int64_t>(g.ws_rows - q0s, INT32_MAX))) - q0);  // wave-uniform
+      if (nq <= 0) return;
+      const int64_t rec0 = (int64_t(split) * g.ws_rows + q0s + q0) * g.Hq + h;
+      if (hf == 0 && ql < nq)
+        *reinterpret_cast<f32x2*>(g.ws + int64_t(g.splits) * g.ws_rows * g.Hq * D + 2 * (rec0 + int64_t(ql) * g.Hq)) =
+            f32x2{m_run[qh], l};
+      constexpr int RP = D + 4, CH = D / 4, PER = 32 * CH / 64;
+      float* wl = reinterpret_cast<float*>(lds) + bwave * 32 * RP;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          *reinterpret_cast<f32x4_t*>(wl + ql * RP + 32 * t + 8 * rr + 4 * hf) =
+              f32x4_t{o[t][qh][4 * rr], o[t][qh][4 * rr + 1], o[t][qh][4 * rr + 2], o[t][qh][4 * rr + 3]};
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int c = lane + 64 * i, qq = c / CH, cc = c % CH;
+        const u32x4 x = *reinterpret_cast<const u32x4*>(wl + qq * RP + 4 * cc);
+        if (qq < nq) store16_wt(g.ws + (rec0 + int64_t(qq) * g.Hq) * D + 4 * cc, x);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    if (g.out_lines) {
+      const int nq = min(32, lq - q0);
+      if (nq <= 0) return;
+      constexpr int RP = D / 2 + 4, CH = D / 8, PER = 32 * CH / 64;
+      uint32_t* wl = reinterpret_cast<uint32_t*>(lds) + bwave * 32 * RP;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          *reinterpret_cast<u32x2*>(wl + ql * RP + 16 * t + 4 * rr + 2 * hf) =
+              u32x2{pack_bf16x2(o[t][qh][4 * rr] * inv, o[t][qh][4 * rr + 1] * inv),
+                    pack_bf16x2(o[t][qh][4 * rr + 2] * inv, o[t][qh][4 * rr + 3] * inv)};
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      uint16_t* ob = g.out + int64_t(q0s + q0) * g.o_st + int64_t(h) * g.o_sh;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int c = lane + 64 * i, qq = c / CH, cc = c % CH;
+        const u32x4 x = *reinterpret_cast<const u32x4*>(wl + qq * RP + 4 * cc);
+        if (qq < nq) store16_wt(ob + int64_t(qq) * g.o_st + 8 * cc, x);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
+    if (qi_lane >= lq) continue;
+    uint16_t* op = g.out + int64_t(q0s + qi_lane) * g.o_st + int64_t(h) * g.o_sh + 4 * hf;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr)
+        *reinterpret_cast<u32x2*>(op + 32 * t + 8 * rr) =
+            u32x2{pack_bf16x2(o[t][qh][4 * rr] * inv, o[t][qh][4 * rr + 1] * inv),
+                  pack_bf16x2(o[t][qh][4 * rr + 2] * inv, o[t][qh][4 * rr + 3] * inv)};
+  }
+}
+
 // Merges the split records of every query of the sequences the prefill kernel took, in split order:
 // O = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), M = max_s m_s; a query no split saw (M = -inf) is zero.
 // One wave per two (query, head) pairs p0 = 2 w, p0 + 1 (pair = query * Hq + head; records of consecutive pairs are
@@ -816,7 +1212,11 @@ extern "C" int nvhip_prefill_attention_bf16(void* out, const void* q, const void
   }
   const dim3 grid(static_cast<unsigned>(blocks + g.dec_extra));
 #define NVHIP_PREFILL_LAUNCH(DD, PG, HBV) hipLaunchKernelGGL((prefill_attention_kernel<DD, PG, HBV>), grid, block, 0, s, g)
-  if (hb == 2 && D == 64 && paged) NVHIP_PREFILL_LAUNCH(64, true, 2);
+  // one sequence over the paged cache (no decode requests in the launch), its key tiles within cache blocks
+  const bool wide = paged && D == 128 && g.lq_skip == 0 && block_size % kBK == 0 && Hkv < (int64_t(1) << 16);
+  if (wide && hb == 2) hipLaunchKernelGGL((prefill_wide_kernel<2>), grid, dim3(kWideThreads), 0, s, g);
+  else if (wide) hipLaunchKernelGGL((prefill_wide_kernel<1>), grid, dim3(kWideThreads), 0, s, g);
+  else if (hb == 2 && D == 64 && paged) NVHIP_PREFILL_LAUNCH(64, true, 2);
   else if (hb == 2 && D == 64) NVHIP_PREFILL_LAUNCH(64, false, 2);
   else if (hb == 2 && paged) NVHIP_PREFILL_LAUNCH(128, true, 2);
   else if (hb == 2) NVHIP_PREFILL_LAUNCH(128, false, 2);

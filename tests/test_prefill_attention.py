@@ -331,3 +331,39 @@ def test_graph_replay_matches_eager():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), rep
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(16, 8), (4, 4), (6, 2), (8, 1)])
+@pytest.mark.parametrize("lq,lk,block_size,causal", [
+    (17, 17, 64, True), (64, 65, 64, True), (65, 128, 256, True), (127, 191, 128, True), (129, 400, 192, True),
+    (300, 300, 256, True), (257, 1281, 64, True), (40, 3000, 256, True), (200, 100, 256, True), (100, 333, 64, False)])
+def test_one_sequence_over_the_cache(lq, lk, block_size, causal, Hq, Hkv):
+    """One sequence over the paged cache whose key tiles of 64 lie in cache blocks: the kernel of 64 queries per wave.
+    Query tiles and key tiles cut short, one to many key tiles per block, key splits (40 over 3000), queries that see
+    nothing, one and two heads per block. block_size 48 (tiles across blocks) runs the other kernel: the same values."""
+    q, kc, vc, bt = paged_case([lq], [lk], block_size, Hq=Hq, Hkv=Hkv, seed=lq + lk + Hq)
+    out, ref = check(q, kc, vc, cu([lq]), cu([lk]), causal, bt)
+    slots = torch.arange(lk)
+    rows = [c[bt[0, slots // block_size].long(), slots % block_size] for c in (kc, vc)]
+    n = (lk + 47) // 48
+    small = [torch.zeros(n * 48, Hkv, 128, dtype=torch.bfloat16) for _ in rows]
+    for s, r in zip(small, rows):
+        s[:lk] = r
+    other, _ = check(q, *(s.view(n, 48, Hkv, 128) for s in small), cu([lq]), cu([lk]), causal,
+                     torch.arange(n, dtype=torch.int32).view(1, n))
+    torch.testing.assert_close(out.float(), other.float(), rtol=2 ** -7, atol=2 ** -9)
+
+
+def test_one_sequence_with_invalid_blocks():
+    """A block-table entry outside the cache stands for keys and values of zero, as in the other kernels."""
+    lq, lk = 130, 700
+    q, kc, vc, bt = paged_case([lq], [lk], 64, seed=3)
+    zeros = torch.zeros(1, *kc.shape[1:], dtype=kc.dtype)
+    ref_bt = bt.clone()
+    ref_bt[0, 2], ref_bt[0, 5] = kc.shape[0], kc.shape[0]
+    bt[0, 2], bt[0, 5] = -1, 1 << 20
+    ref = oracle.varlen_attention(q, torch.cat([kc, zeros]), torch.cat([vc, zeros]), cu([lq]), cu([lk]), 128 ** -0.5,
+                                  True, ref_bt)
+    out = flash_attn_varlen_func(q.to(DEV), kc.to(DEV), vc.to(DEV), lq, cu([lq]).to(DEV), lk, cu([lk]).to(DEV),
+                                 128 ** -0.5, True, bt.to(DEV)).cpu()
+    torch.testing.assert_close(out.float(), ref.float(), rtol=1.6e-2, atol=1e-2)
