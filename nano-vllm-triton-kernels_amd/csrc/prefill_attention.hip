@@ -78,6 +78,7 @@ struct PrefillArgs {
   // dec_extra > 0 (dec.halves): the short sequences' (sequence, kv head) pairs are cut in two; the blocks above
   // run the first halves, dec_extra blocks appended to the grid (one per pair of the call) the second halves
   int dec_extra;
+  int plan;       // number of sequences (at most 64) when the blocks find their tile with block_plan, else 0
   int out_lines;  // out 16-byte aligned with strides in whole 16-byte pieces: the output goes out in whole lines
   DecodeArgs dec;
 };
@@ -92,6 +93,60 @@ __device__ __forceinline__ int64_t key_row(const PrefillArgs& g, int k0s, int j,
   if constexpr (!PAGED) return int64_t(k0s + j) * st + int64_t(kvh) * D;
   if (blk < 0 || blk >= g.num_blocks) return -1;
   return ((int64_t(blk) * g.bs + j % g.bs) * g.Hkv + kvh) * D;
+}
+
+// Which sequence and query tile block `item` of a ragged launch's (sequence, tile) pairs is, for calls of up to 64 sequences:
+// first the query tiles of the sequences that the prefill kernel takes, the latest (most keys) first across all of
+// them, then the sequences left to the decode attention (tile -1), then nothing (false): what the grid, sized for the
+// longest sequence, holds beyond that. Every wave computes it from the sequence bounds, one sequence per lane. Without
+// it a mixed step's prompt chunk started behind the decode requests' blocks, its last tiles two rounds late, and the
+// ends of a ragged batch's grid came between its tiles.
+struct Plan {
+  int b, qt, q0, lq, k0, lk;
+};
+__device__ __forceinline__ int nth_bit(uint64_t mask, int n) {  // position of set bit n (it exists)
+  const int lane = threadIdx.x % 64;
+  const int below = __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0));
+  return __builtin_ctzll(__ballot(((mask >> lane) & 1) != 0 && below == n));
+}
+template <int BQ>
+__device__ __forceinline__ bool block_plan(const PrefillArgs& g, int item, Plan& p) {
+  const int lane = threadIdx.x % 64;
+  const bool in = lane < g.plan;
+  const int q0 = in ? g.cu_q[lane] : 0, k0 = in ? g.cu_k[lane] : 0;
+  const int lq = (in ? g.cu_q[lane + 1] : 0) - q0, lk = (in ? g.cu_k[lane + 1] : 0) - k0;
+  const bool brief = lq >= 1 && lq <= g.lq_skip;
+  const int tiles = brief ? 0 : min((lq + BQ - 1) / BQ, g.qtiles);  // < 256
+  auto from = [&](int level) {  // tiles at or above this level, of all sequences: the bits of the lanes' counts
+    const int n = max(tiles - level, 0);
+    int sum = 0;
+#pragma unroll
+    for (int bit = 0; bit < 8; ++bit) sum += __builtin_popcountll(__ballot((n >> bit) & 1)) << bit;
+    return sum;
+  };
+  const int total = from(0);
+  uint64_t mask;
+  int n;
+  if (item < total) {
+    int lo = 0, hi = g.qtiles;  // from(lo) > item >= from(hi)
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) / 2;
+      if (from(mid) > item) lo = mid;
+      else hi = mid;
+    }
+    p.qt = lo;
+    n = item - from(lo + 1);
+    mask = __ballot(tiles > lo);
+  } else {
+    p.qt = -1;
+    n = item - total;
+    mask = __ballot(brief);
+    if (n >= __builtin_popcountll(mask)) return false;
+  }
+  p.b = nth_bit(mask, n);
+  p.q0 = __builtin_amdgcn_readlane(q0, p.b), p.lq = __builtin_amdgcn_readlane(lq, p.b);
+  p.k0 = __builtin_amdgcn_readlane(k0, p.b), p.lk = __builtin_amdgcn_readlane(lk, p.b);
+  return true;
 }
 
 // HB q heads of one kv head per block (4 waves each, sharing the K/V tiles in LDS).
@@ -133,24 +188,33 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
     }
     return;
   }
-  int grp, ci;
-  if (nblk % 8 == 0 && (nblk / 8) % ntile == 0) {
-    const int gx = nblk / 8 / ntile, r = blockIdx.x / 8;
-    grp = (r % gx) * 8 + blockIdx.x % 8;
-    ci = r / gx;
+  int b, hg, qt, split, q0s, lq, k0s, lk;
+  if (g.plan) {  // (no key splits; the head groups divide evenly over the XCDs)
+    const int sub = g.nhg / 8, r = blockIdx.x / 8;
+    Plan p;
+    if (!block_plan<kBQ>(g, r / sub, p)) return;
+    hg = r % sub * 8 + int(blockIdx.x) % 8;
+    b = p.b, qt = max(p.qt, 0), split = 0, q0s = p.q0, lq = p.lq, k0s = p.k0, lk = p.lk;
   } else {
-    grp = blockIdx.x % ngrp;
-    ci = blockIdx.x / ngrp;
+    int grp, ci;
+    if (nblk % 8 == 0 && (nblk / 8) % ntile == 0) {
+      const int gx = nblk / 8 / ntile, r = blockIdx.x / 8;
+      grp = (r % gx) * 8 + blockIdx.x % 8;
+      ci = r / gx;
+    } else {
+      grp = blockIdx.x % ngrp;
+      ci = blockIdx.x / ngrp;
+    }
+    qt = g.qtiles - 1 - ci / g.splits, split = ci % g.splits;
+    b = grp / g.nhg, hg = grp % g.nhg;
+    q0s = g.cu_q[b], lq = g.cu_q[b + 1] - q0s;
+    k0s = g.cu_k[b], lk = g.cu_k[b + 1] - k0s;
   }
-  const int qt = g.qtiles - 1 - ci / g.splits, split = ci % g.splits;
-  const int b = grp / g.nhg, hg = grp % g.nhg;
   const int h = hg * HB + int(threadIdx.x) / kHeadThreads, kvh = (hg * HB) / g.G;
-  const int q0s = g.cu_q[b], lq = g.cu_q[b + 1] - q0s;
-  const int k0s = g.cu_k[b], lk = g.cu_k[b + 1] - k0s;
   if (lq >= 1 && lq <= g.lq_skip) {  // the paged decode attention takes this sequence (the whole block: b is uniform)
-    // one block per (sequence, kv head) runs the decode attention of the pair (the whole block: b, hg, ci uniform)
+    // one block per (sequence, kv head) runs the decode attention of the pair (the whole block: b, hg, qt uniform)
     if constexpr (PAGED) {
-      if (g.dec_inline && ci == 0 && (hg * HB) % g.G == 0) {
+      if (g.dec_inline && (g.plan || qt == g.qtiles - 1) && split == 0 && (hg * HB) % g.G == 0) {
         const int pair = b * g.Hkv + hg * HB / g.G, bid = g.dec.halves ? 2 * pair : pair;
         if (g.dec.bs % 32 == 0) decode_block<D, 16, true, false, true>(g.dec, bid, reinterpret_cast<unsigned char*>(lds));
         else decode_block<D, 16, false, false, true>(g.dec, bid, reinterpret_cast<unsigned char*>(lds));
@@ -1210,6 +1274,12 @@ extern "C" int nvhip_prefill_attention_bf16(void* out, const void* q, const void
                                  dws ? workspace_size - off : 0, s);
     }
   }
+  // block_plan: lanes for sequences, eighths of the head groups for XCDs. 24 prompts of 30 .. 2100 tokens 259 -> 209-217
+  // us, 48 decode requests and a chunk of 464 queries 87 -> 70, 7 and a chunk of 2000 over 5000 cached keys 486 -> 278 (q/k
+  // norm kernel included); the plan takes a block ~0.5 us, and sequences of one length are in its order already (4 x
+  // 2048 tokens 81 us without, 83 with it).
+  const bool ragged = total_q < num_seqs * max_seqlen_q;
+  g.plan = ragged && num_seqs <= 64 && g.nhg % 8 == 0 && g.splits == 1 && qtiles < 256 ? int(num_seqs) : 0;
   const dim3 grid(static_cast<unsigned>(blocks + g.dec_extra));
 #define NVHIP_PREFILL_LAUNCH(DD, PG, HBV) hipLaunchKernelGGL((prefill_attention_kernel<DD, PG, HBV>), grid, block, 0, s, g)
   // one sequence over the paged cache (no decode requests in the launch), its key tiles within cache blocks
