@@ -382,8 +382,9 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_nt(const Mfm
       float gf[8], uf[8], o[8];
       unpack8(gv, gf);
       unpack8(uv, uf);
+      silu_bf16_n(gf, o);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = silu_bf16(gf[e]) * uf[e];
+      for (int e = 0; e < 8; ++e) o[e] *= uf[e];
       const u32x4 v = pack8(o);
       uint16_t* d = g.c + int64_t(m) * g.scm + n;
       if (n + 8 <= n2 && (reinterpret_cast<uintptr_t>(d) & 15) == 0) {
@@ -634,12 +635,16 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_stream_nt(const M
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           float v[4];
+          if constexpr (SILU) {
+            float gate[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if constexpr (SILU)
-              v[e] = silu_bf16(round_bf16(acc[i + t][j][e])) * round_bf16(acc[i + t][j + FN / 2][e]);
-            else
-              v[e] = acc[i + t][j][e];
+            for (int e = 0; e < 4; ++e) gate[e] = round_bf16(acc[i + t][j][e]);
+            silu_bf16_n(gate, v);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] *= round_bf16(acc[i + t][j + FN / 2][e]);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = acc[i + t][j][e];
           }
           w[t][0] = pack_bf16x2(v[0], v[1]);
           w[t][1] = pack_bf16x2(v[2], v[3]);

@@ -355,3 +355,15 @@ def test_fp32_values_without_parts(M, N, K, nmajor, prec):
     assert (got - want).norm() / want.norm() < math.sqrt(K) * 2.0 ** -24
     tiny = c[11, cols].double()  # denormal times normal: fp32's own spacing there is 2^-149
     torch.testing.assert_close(tiny, ref[11, cols], rtol=1e-5, atol=K * 2.0 ** -149)
+
+
+@pytest.mark.parametrize("M", [256, 2304])   # the staged and the streaming kernel's epilogue
+def test_fused_silu_at_every_finite_gate(M):
+    """One-hot rows of x pick single weights, so the gates are every finite bf16 value: the fused epilogue's silu is
+    bitwise the unfused kernel's (torch's formula with the exact exp and divide)."""
+    values = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(1024, 64).clone()
+    values[~values.isfinite()] = 0.0
+    w = torch.cat([values, torch.ones_like(values)]).to(DEV)
+    x = torch.eye(64, dtype=torch.bfloat16, device=DEV).repeat(M // 64, 1)
+    gate = values.t().repeat(M // 64, 1).to(DEV)
+    assert torch.equal(matmul_silu_and_mul(x, w), silu_and_mul(torch.cat([gate, torch.ones_like(gate)], dim=1)))
