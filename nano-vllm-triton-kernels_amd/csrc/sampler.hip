@@ -42,7 +42,11 @@ __device__ __forceinline__ void merge(Best& b, float v, int64_t i) {
   if (beats(v, i, b.v, b.i)) b.v = v, b.i = i;
 }
 
-// Best of elements [lo, hi) of a row (lo a multiple of 8 when VEC), over the block; the result in thread 0.
+// Best of elements [lo, hi) of a row (lo a multiple of 8 when VEC), over the block; the result in thread 0. Whole
+// 16-byte chunks are compared by their maximum: a thread keeps the first chunk whose maximum is the largest and whether
+// it saw a NaN, ~3 VALU instructions per logit instead of ~7 for a (value, 64-bit index) pair per logit, and looks up
+// the element in that chunk at the end; a thread that saw a NaN goes over its chunks again in the full order. 250 x
+// 151936 (76 MB) 21.5 -> 17.2 us, 32 x 151936 6.6 -> 5.5 us.
 template <bool VEC>
 __device__ __forceinline__ Best block_best(const uint16_t* row, int64_t lo, int64_t hi) {
   const int tid = threadIdx.x;
@@ -50,25 +54,46 @@ __device__ __forceinline__ Best block_best(const uint16_t* row, int64_t lo, int6
   int64_t tail = lo;
   if constexpr (VEC) {
     const int64_t c0 = lo / 8, c1 = hi / 8;  // whole 16-byte chunks
-    const u32x4* rv = reinterpret_cast<const u32x4*>(row);
-    int64_t c = c0 + tid;
-    for (; c + 3 * kThreads < c1; c += 4 * kThreads) {
-      u32x4 q[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) q[u] = rv[c + u * kThreads];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        float f[8];
-        unpack8(q[u], f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) take_later(b, f[e], (c + u * kThreads) * 8 + e);
-      }
-    }
-    for (; c < c1; c += kThreads) {
+    const u32x4* rv = reinterpret_cast<const u32x4*>(row) + c0;
+    const int n = int(c1 - c0);  // of this slice
+    constexpr int U = 8;
+    int best = -1;
+    bool nan = false;
+    auto take = [&](const u32x4& q, int c) {
       float f[8];
-      unpack8(rv[c], f);
+      unpack8(q, f);
+      float m = f[0];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) take_later(b, f[e], c * 8 + e);
+      for (int e = 1; e < 8; ++e) m = fmaxf(m, f[e]);
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) nan |= __builtin_isunordered(f[e], f[e + 1]);
+      if (m > b.v) b.v = m, best = c;
+    };
+    int c = tid;
+    for (; c + (U - 1) * kThreads < n; c += U * kThreads) {
+      u32x4 q[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) q[u] = rv[c + u * kThreads];
+#pragma unroll
+      for (int u = 0; u < U; ++u) take(q[u], c + u * kThreads);
+    }
+    for (; c < n; c += kThreads) take(rv[c], c);
+    if (nan) {
+      b = Best{-INFINITY, INT64_MAX};
+      for (c = tid; c < n; c += kThreads) {
+        float f[8];
+        unpack8(rv[c], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) take_later(b, f[e], (c0 + c) * 8 + e);
+      }
+    } else if (best >= 0) {
+      float f[8];
+      unpack8(rv[best], f);
+      int at = 7;
+#pragma unroll
+      for (int e = 6; e >= 0; --e)
+        if (f[e] == b.v) at = e;
+      b.i = (c0 + best) * 8 + at;
     }
     tail = c1 * 8;
   }
@@ -117,9 +142,10 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(int64_t* __restrict__ 
   if (l == 0) out[blockIdx.x] = b.i < n ? b.i : 0;
 }
 
-// slices per row: enough blocks for every CU (rows * S >= 512), slices of at least 4096 elements, S <= 64
+// slices per row: enough blocks for every CU to hold its eight (rows * S >= 2048), slices of at least 4096 elements,
+// S <= 64
 int argmax_slices(int64_t rows, int64_t n) {
-  int64_t s = (512 + rows - 1) / rows;
+  int64_t s = (2048 + rows - 1) / rows;
   s = std::min<int64_t>(s, (n + 4095) / 4096);
   return int(std::max<int64_t>(1, std::min<int64_t>(s, 64)));
 }
