@@ -95,10 +95,10 @@ __device__ __forceinline__ int64_t key_row(const PrefillArgs& g, int k0s, int j,
   return ((int64_t(blk) * g.bs + j % g.bs) * g.Hkv + kvh) * D;
 }
 
-// Which sequence and query tile block `item` of a ragged launch's (sequence, tile) pairs is, for calls of up to 64 sequences:
-// first the query tiles of the sequences that the prefill kernel takes, the latest (most keys) first across all of
-// them, then the sequences left to the decode attention (tile -1), then nothing (false): what the grid, sized for the
-// longest sequence, holds beyond that. Every wave computes it from the sequence bounds, one sequence per lane. Without
+// Which sequence and query tile block `item` of a ragged launch's (sequence, tile) pairs is, for calls of up to 64
+// sequences: first the query tiles of the sequences that the prefill kernel takes, the latest (most keys) first across
+// all of them, then the sequences left to the decode attention (tile -1), then nothing (false): what the grid, sized
+// for the longest sequence, holds beyond that. Every wave computes it from the sequence bounds, one sequence per lane. Without
 // it a mixed step's prompt chunk started behind the decode requests' blocks, its last tiles two rounds late, and the
 // ends of a ragged batch's grid came between its tiles.
 struct Plan {
@@ -1274,10 +1274,10 @@ extern "C" int nvhip_prefill_attention_bf16(void* out, const void* q, const void
                                  dws ? workspace_size - off : 0, s);
     }
   }
-  // block_plan: lanes for sequences, eighths of the head groups for XCDs. 24 prompts of 30 .. 2100 tokens 259 -> 209-217
-  // us, 48 decode requests and a chunk of 464 queries 87 -> 70, 7 and a chunk of 2000 over 5000 cached keys 486 -> 278 (q/k
-  // norm kernel included); the plan takes a block ~0.5 us, and sequences of one length are in its order already (4 x
-  // 2048 tokens 81 us without, 83 with it).
+  // block_plan: lanes for sequences, eighths of the head groups for XCDs. 24 prompts of 30 .. 2100 tokens 259 ->
+  // 209-217 us, 48 decode requests and a chunk of 464 queries 87 -> 70, 7 and a chunk of 2000 over 5000 cached keys
+  // 486 -> 278 (q/k norm kernel included); the plan takes a block ~0.5 us, and sequences of one length are in its
+  // order already (4 x 2048 tokens 81 us without, 83 with it).
   const bool ragged = total_q < num_seqs * max_seqlen_q;
   g.plan = ragged && num_seqs <= 64 && g.nhg % 8 == 0 && g.splits == 1 && qtiles < 256 ? int(num_seqs) : 0;
   const dim3 grid(static_cast<unsigned>(blocks + g.dec_extra));

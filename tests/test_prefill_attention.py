@@ -333,6 +333,31 @@ def test_graph_replay_matches_eager():
         assert torch.equal(out, eager), rep
 
 
+@pytest.mark.parametrize("Hq,Hkv,D", [(16, 8, 128), (32, 8, 128), (16, 8, 64)])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("lq", [
+    [1, 300], [64, 65, 63, 0, 129, 1], [0, 0, 200, 1, 1, 17, 0], [20] * 63 + [321], [1, 2, 8, 9] * 15 + [257, 0, 0, 128]])
+def test_ragged_batches_in_plan_order(lq, paged, Hq, Hkv, D):
+    """Up to 64 sequences of different lengths: the blocks find their tiles from the sequence bounds. Empty sequences
+    first, last and between, tiles cut short, decode requests and short runs behind the long sequences (the cache), a
+    full wave of sequences. With empty sequences added until there are more than 64 the blocks take them in grid order:
+    every query of the prefill kernel has the same bits."""
+    lk = [n + 37 * (i % 3) if paged and n else n for i, n in enumerate(lq)]
+    more = 65 - len(lq)
+    if paged:
+        q, k, v, bt = paged_case(lq, lk, 64, Hq=Hq, Hkv=Hkv, D=D, seed=sum(lq))
+        bt_more = torch.cat([bt, torch.full((more, bt.shape[1]), -1, dtype=torch.int32)])
+    else:
+        _, q, k, v = contiguous_case(lq, Hq=Hq, Hkv=Hkv, D=D, seed=sum(lq))
+        bt = bt_more = None
+    out, _ = check(q, k, v, cu(lq), cu(lk), True, bt)
+    other, _ = check(q, k, v, cu(lq + [0] * more), cu(lk + [0] * more), True, bt_more)
+    skip = 16 // (Hq // Hkv) if paged else 0  # those rows are the decode attention's, its splits by the call's size
+    for i, n in enumerate(lq):
+        if n > skip:
+            assert torch.equal(out[sum(lq[:i]):sum(lq[:i + 1])], other[sum(lq[:i]):sum(lq[:i + 1])]), i
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(16, 8), (4, 4), (6, 2), (8, 1)])
 @pytest.mark.parametrize("lq,lk,block_size,causal", [
     (17, 17, 64, True), (64, 65, 64, True), (65, 128, 256, True), (127, 191, 128, True), (129, 400, 192, True),
