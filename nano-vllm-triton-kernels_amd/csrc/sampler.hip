@@ -7,8 +7,8 @@
 //
 // Each thread visits its chunks in increasing index order, so inside a thread "strictly larger" replaces the running
 // best (no index comparison); threads, waves and blocks merge with the full order. With a workspace the row is split
-// over S blocks (S * rows up to ~2048: several blocks per CU) whose (value, index) results a second launch merges per
-// row; without one, one block per row. At 32 x 151936 (a decode step of Qwen3-0.6B) the split form takes 5.5 us and
+// over S blocks (S * rows >= 512: every CU gets work) whose (value, index) results a second launch merges per
+// row; without one, one block per row. At 32 x 151936 (a decode step of Qwen3-0.6B) the split form takes 5.8 us and
 // the merge 4; torch's bf16 -> fp32 copy and ArgMaxOps took 6.6 + 59.8 us.
 #include <algorithm>
 #include <cfloat>
@@ -45,7 +45,7 @@ __device__ __forceinline__ void merge(Best& b, float v, int64_t i) {
 // 16-byte chunks are compared by their maximum: a thread keeps the first chunk whose maximum is the largest and whether
 // it saw a NaN, ~3 VALU instructions per logit instead of ~7 for a (value, 64-bit index) pair per logit, and looks up
 // the element in that chunk at the end; a thread that saw a NaN goes over its chunks again in the full order. 250 x
-// 151936 (76 MB) 21.5 -> 17.2 us, 32 x 151936 6.6 -> 5.5 us.
+// 151936 (76 MB) 21.5 -> 15.5 us, 32 x 151936 6.6 -> 5.8 us.
 template <bool VEC>
 __device__ __forceinline__ Best block_best(const uint16_t* row, int64_t lo, int64_t hi) {
   const int tid = threadIdx.x;
@@ -141,10 +141,9 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(int64_t* __restrict__ 
   if (l == 0) out[blockIdx.x] = b.i < n ? b.i : 0;
 }
 
-// slices per row: enough blocks for every CU to hold its eight (rows * S >= 2048), slices of at least 4096 elements,
-// S <= 64
+// slices per row: enough blocks for every CU (rows * S >= 512), slices of at least 4096 elements, S <= 64
 int argmax_slices(int64_t rows, int64_t n) {
-  int64_t s = (2048 + rows - 1) / rows;
+  int64_t s = (512 + rows - 1) / rows;
   s = std::min<int64_t>(s, (n + 4095) / 4096);
   return int(std::max<int64_t>(1, std::min<int64_t>(s, 64)));
 }
