@@ -705,7 +705,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
   const uint32_t row_bytes = uint32_t(g.Hkv) * D * 2;
   uint32_t kofs[4], vofs[4];
   const int lr = lane / 16, lc = lane % 16;
-  auto offsets = [&](int v_rows, int k_rows) {  // rows of the tiles that exist; past them the last one again
+  auto offsets = [&](int v_rows, int k_rows) {  // rows of the tiles that exist; past them the last one again (K rows
+                                                // there are masked, V rows zeroed by mask())
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int row = 4 * (bwave + 4 * j) + lr;
@@ -789,8 +790,19 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
     return __builtin_bit_cast(bf16x8_t, u32x4{lo[0], lo[1], hi[0], hi[1]});
   };
   using Scores = f32x16_t[2][2];  // [u][qh]
-  auto mask = [&](Scores& s, int kt0) {  // where the tile at kt0 needs it
+  // Masks the scores of the tile at kt0 where it needs it, in front of the barrier that hands out its V rows (slot; one
+  // event's loads were issued after them). Behind the last key those are copies of its row, and 0 times an infinity there
+  // would be NaN: each wave zeroes what it loaded itself.
+  auto mask = [&](Scores& s, int kt0, int slot) {
     if (kt0 + kBK <= lk && (!g.causal || kt0 + kBK - 1 <= diag + wave_q0)) return;
+    if (kt0 + kBK > lk) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * (bwave + 4 * j) + lr >= lk - kt0)
+          *reinterpret_cast<u32x4*>(lds + (NK + slot) * TILE + j * 4096 + bwave * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
 #pragma unroll
     for (int qh = 0; qh < 2; ++qh) {
       const int lim = min(lk - 1, g.causal ? diag + wave_q0 + 32 * qh + ql : lk - 1) - kt0 - 4 * hf;
@@ -832,7 +844,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
   static_for<32>([&](auto xc) { scores_mfma(sa, xc); });
   next_slot(k_slot, NK);
   asm volatile("s_nop 15\n\ts_nop 15" : "+v"(sa[0][0]), "+v"(sa[0][1]), "+v"(sa[1][0]), "+v"(sa[1][1]));
-  mask(sa, kt0);
+  mask(sa, kt0, v_slot);
   static_for<32>([&](auto kc) { max_step(sa, kc); });
   max_done();
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LOADS) : "memory");
@@ -897,7 +909,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
         // K(next + 1) and V(next) have landed, and everybody has read K(next) and the V before this one: their slots
         // are free
         asm volatile("" : "+v"(sn[0][0]), "+v"(sn[0][1]), "+v"(sn[1][0]), "+v"(sn[1][1]));
-        mask(sn, kt0 + kBK);
+        mask(sn, kt0 + kBK, v_slot + 1 == NV ? 0 : v_slot + 1);
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS) : "memory");
         next_load();
       }

@@ -392,3 +392,23 @@ def test_one_sequence_with_invalid_blocks():
     out = flash_attn_varlen_func(q.to(DEV), kc.to(DEV), vc.to(DEV), lq, cu([lq]).to(DEV), lk, cu([lk]).to(DEV),
                                  128 ** -0.5, True, bt.to(DEV)).cpu()
     torch.testing.assert_close(out.float(), ref.float(), rtol=1.6e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(16, 8), (4, 4)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("lq,lk,block_size", [(17, 17, 64), (40, 127, 64), (200, 333, 256), (130, 3001, 256),
+                                              (40, 127, 48)])
+def test_infinite_value_of_the_last_key(lq, lk, block_size, causal, Hq, Hkv):
+    """An infinity in the last key's V row, with key tiles of 64 cut short behind it (nothing past the last key takes
+    part in a sum): the queries that see that key get the infinity, in every kernel of one sequence over the cache,
+    with and without key splits; the other dims are as they are without it."""
+    q, kc, vc, bt = paged_case([lq], [lk], block_size, Hq=Hq, Hkv=Hkv, seed=lq + lk)
+    out, _ = check(q, kc, vc, cu([lq]), cu([lk]), causal, bt)
+    blk, slot = bt[0, (lk - 1) // block_size].long(), (lk - 1) % block_size
+    vc[blk, slot, :, 5], vc[blk, slot, :, 77] = float("inf"), float("-inf")
+    got = flash_attn_varlen_func(q.to(DEV), kc.to(DEV), vc.to(DEV), lq, cu([lq]).to(DEV), lk, cu([lk]).to(DEV),
+                                 128 ** -0.5, causal, bt.to(DEV)).cpu()
+    rows = slice(lq - 1, lq) if causal else slice(0, lq)
+    assert torch.all(got[rows, :, 5] == float("inf")) and torch.all(got[rows, :, 77] == float("-inf"))
+    dims = [d for d in range(128) if d not in (5, 77)]
+    assert torch.equal(got[:, :, dims], out[:, :, dims])
