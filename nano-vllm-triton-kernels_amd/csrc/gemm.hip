@@ -12,7 +12,7 @@
 //   gemm_stream_nt bf16, K-contiguous A and B, when there are more tiles than one round on the CUs: persistent blocks,
 //                  memory -> LDS loads, 16x16x32 MFMA; the same bits.
 //   gemm_skinny    bf16 with M <= 32, same layout: 16 columns per block, K split over 8 waves, 16x16x32 MFMA.
-//   gemm_split_f32 fp32, A K-contiguous, B K- or N-contiguous: exact bf16 parts on the bf16 MFMA, fp32 sums.
+//   gemm_mfma_f32  fp32, A K-contiguous, B K- or N-contiguous: 32x32x2 fp32 MFMA (exact products, fp32 sums).
 //   gemm_generic   any dtype/strides/precision: 64x64 tile, 4x4 outputs per thread, fp32 FMA.
 #include <type_traits>
 #include <utility>
@@ -1177,29 +1177,17 @@ __global__ __launch_bounds__(512) void gemm_skinny_norm(const NormMfmaArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// fp32 kernel on the bf16 matrix cores. A is K-contiguous; B is either K-contiguous (W [N, K], B = W.t()) or
-// N-contiguous ([K, N]). Every fp32 value is the exact sum of three bf16 parts (each the rest rounded to nearest: 3 x 8
-// significant bits), a tf32 value (TF32: inputs rounded to a 10-bit mantissa first) of two, so a product is a sum of
-// exact bf16 products, which the MFMA adds in fp32: for tf32 all four, for fp32 the six down to 2^-16 of the whole; the
-// three left out (parts 2 x 3, 3 x 2, 3 x 3) are below 2^-24 of it, at random signs. The bf16 cores do 16 times the
-// flops of the fp32 ones, so six products still take less time, and one rounding of the sum per 32 k and product
-// instead of one per 2 k loses less: error against 64-bit sums (2-norm, normal A and B) at K = 4096 / 1000 / 64 1.00e-6
-// / 4.8e-7 / 0.9e-7, 1.15e-6 / 5.6e-7 / 1.5e-7 with v_mfma_f32_32x32x2_f32; tf32 8.0e-7 / 3.8e-7 / 0.7e-7 against
-// 1.14e-6 / 5.5e-7 / 1.3e-7.
-//
-// BM x BN block tile, k-tile 32, each wave (BM / WAVES_M) x (BN / WAVES_N) outputs as 16x16x32 MFMA tiles (operands
-// swapped as in the bf16 kernels). A thread brings 8 consecutive k of a row (a column of an N-contiguous B) to
-// registers, splits them and writes one 16-byte chunk per part plane; a plane's rows are 64 bytes, chunk c of row r at
-// chunk c ^ ((r >> 2) & 3), so that 16 rows fall on distinct banks. Two LDS stages; a chunk of the next k-tile is split
-// and stored, and the k-tile after that requested into its registers, in front of each row of MFMAs. What bounds it is
-// the matrix cores at the clock that they keep under this load (1.25 PFLOP/s of bf16 at 4096^3) and, for tf32 and the
-// smaller tiles, the splitting (about 8 VALU instructions per element staged).
-// 4096^3 (N- / K-contiguous B) against the fp32 MFMA kernel: 988 -> 705 / 973 -> 661 us, tf32 1072 -> 562 / 1112 ->
-// 520; 1024^3 79 -> 32 / 97 -> 28 us; nine products 871 us and no smaller an error.
-//
-// Parts that bf16 cannot hold, and what the split does not carry: a block that has met an infinity, a NaN, a value that
-// rounds past the largest bf16, a nonzero one below 2^-110 (its last part would end below the smallest bf16
-// denormal), or a result that is not finite, computes its tile again with fp32 MFMAs on the values themselves.
+// fp32 MFMA kernel: v_mfma_f32_32x32x2_f32 forms exact fp32 products and accumulates them in fp32 (precision
+// "ieee"); with TF32 every input is first rounded to tf32. A is K-contiguous; B is either K-contiguous (W [N, K],
+// B = W.t()) or N-contiguous ([K, N]). BM x BN block tile of WAVES_M x WAVES_N waves, each owning (BM / WAVES_M) x
+// (BN / WAVES_N) outputs as 32x32 MFMA tiles (operands swapped as in the bf16 kernel), k-tile 32. LDS holds both
+// operands k-major ([k][m], [k][n]) with row pitches of BM + 32 and BN + 32 floats (32 mod 64 banks), so the two
+// half-waves of a fragment read (rows k and k+1, 32 consecutive floats each) hit disjoint bank halves. Global loads
+// are 16 bytes: 4 consecutive k of one row of A / W (8 lanes cover one row's 128 bytes), or 4 consecutive n of one
+// row of B. The next k-tile is loaded into registers at the start of the current one and stored into the other LDS
+// stage halfway through its MFMAs (stores after the last MFMA left the matrix cores idle during them). 4096^3:
+// 256x256 tiles with 16 waves (4 per SIMD) 1107 us, 128x128 with 8 waves 1167 us, 128x128 with 4 waves and the
+// stores at the end 1434 us.
 struct F32Args {
   float* c;
   const float* a;
@@ -1209,187 +1197,268 @@ struct F32Args {
 };
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool B_NMAJOR, bool TF32>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_split_f32(const F32Args g) {
-  constexpr int NT = 64 * WAVES_M * WAVES_N, BK = 32, P = TF32 ? 2 : 3;  // P: parts of a value
-  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 16, FN = WN / 16;
-  constexpr int CA = BM * 4 / NT, CB = BN * 4 / NT;  // 8-element chunks per thread and k-tile
-  static_assert(CA * NT == BM * 4 && CB * NT == BN * 4, "whole chunks per thread");
-  constexpr int PA = BM * 64, PB = BN * 64, STAGE = P * (PA + PB);  // bytes: planes of A rows, then of B rows
-  static_assert(2 * STAGE <= 160 * 1024 - 1024, "LDS");
-  __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_mfma_f32(const F32Args g) {
+  constexpr int NT = 64 * WAVES_M * WAVES_N, BK = 32, PA = BM + 32, PB = BN + 32;
+  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 32, FN = WN / 32;
+  constexpr int CHA = BM * BK / 4 / NT, CHB = BN * BK / 4 / NT;  // 16-byte chunks per thread per k-tile
+  static_assert(FM >= 1 && FN >= 1 && CHA >= 1 && CHB >= 1 && CHA * NT * 4 == BM * BK && CHB * NT * 4 == BN * BK,
+                "tile shape");
+  __shared__ __attribute__((aligned(16))) float lds[2][BK * (PA + PB)];  // [stage][A k-major | B k-major]
   int pid_m, pid_n;
   tile_coords(blockIdx.x, g.M, g.N, BM, BN, pid_m, pid_n);
   const int m0 = pid_m * BM, n0 = pid_n * BN;
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int64_t sbk = B_NMAJOR ? g.sbk : 1, sbn = B_NMAJOR ? 1 : g.sbn;
 
-  // chunk c < CA: row (tid + NT c) / 4 of the A tile, k 8 ((tid + NT c) % 4) .. +8; else of the B tile, an
-  // N-contiguous B with its columns along the lanes
-  const float* src[CA + CB];
-  int dst[CA + CB], kofs[CA + CB];
+  // K-major chunks (A, and B when K-contiguous): chunk c covers row c / 8, k = 4 * (c % 8) .. +4
+  const float* asrc[CHA];
+  const float* bsrc[CHB];
+  int arow[CHA], akc[CHA], brow[CHB], bkc[CHB];
 #pragma unroll
-  for (int i = 0; i < CA + CB; ++i) {
-    const bool is_a = i < CA;
-    const int c = tid + NT * (is_a ? i : i - CA);
-    const int row = !is_a && B_NMAJOR ? c % BN : c / 4, kc = !is_a && B_NMAJOR ? c / BN : c % 4;
-    src[i] = is_a ? g.a + int64_t(min(m0 + row, g.M - 1)) * g.sam : g.b + int64_t(min(n0 + row, g.N - 1)) * sbn;
-    dst[i] = (is_a ? 0 : P * PA) + row * 64 + (kc ^ ((row >> 2) & 3)) * 16;
-    kofs[i] = 8 * kc;
+  for (int i = 0; i < CHA; ++i) {
+    const int c = tid + NT * i;
+    arow[i] = c / 8;
+    akc[i] = 4 * (c % 8);
+    asrc[i] = g.a + int64_t(min(m0 + arow[i], g.M - 1)) * g.sam + akc[i];
   }
-  float r[CA + CB][8];
-  auto gload = [&](int i, int k0) {  // K % 4 == 0. Past K: zeros of A, and the last values of B again
-    if (i >= CA && B_NMAJOR) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r[i][e] = src[i][int64_t(min(k0 + kofs[i] + e, g.K - 1)) * sbk];
-      return;
+  for (int i = 0; i < CHB; ++i) {
+    const int c = tid + NT * i;
+    if constexpr (B_NMAJOR) {  // chunk c covers k row c / (BN / 4), n = 4 * (c % (BN / 4)) .. +4 (clamped inside N)
+      brow[i] = c / (BN / 4);
+      bkc[i] = 4 * (c % (BN / 4));
+      bsrc[i] = g.b + min(n0 + bkc[i], g.N - 4);
+    } else {
+      brow[i] = c / 8;
+      bkc[i] = 4 * (c % 8);
+      bsrc[i] = g.b + int64_t(min(n0 + brow[i], g.N - 1)) * g.sbn + bkc[i];
     }
+  }
+  f32x4_t ra[CHA], rb[CHB];
+  auto gload = [&](int k0) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int k = k0 + kofs[i] + 4 * h;
-      f32x4_t v{0, 0, 0, 0};
-      if (i >= CA || k < g.K) v = *reinterpret_cast<const f32x4_t*>(src[i] + min(k, g.K - 4));
+    for (int i = 0; i < CHA; ++i)
+      ra[i] = (k0 + akc[i] < g.K) ? *reinterpret_cast<const f32x4_t*>(asrc[i] + k0) : f32x4_t{0, 0, 0, 0};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) r[i][4 * h + e] = v[e];
+    for (int i = 0; i < CHB; ++i) {
+      if constexpr (B_NMAJOR)
+        rb[i] = (k0 + brow[i] < g.K) ? *reinterpret_cast<const f32x4_t*>(bsrc[i] + int64_t(k0 + brow[i]) * g.sbk)
+                                     : f32x4_t{0, 0, 0, 0};
+      else
+        rb[i] = (k0 + bkc[i] < g.K) ? *reinterpret_cast<const f32x4_t*>(bsrc[i] + k0) : f32x4_t{0, 0, 0, 0};
     }
   };
-  uint32_t least = 0xffffffffu, most = 0;  // of the values staged: |x| - 1 (0 wraps to the largest), and |x|, as bits
-  auto lstore = [&](int i, int stage) {
-    u32x4 w[P];
+  auto tf = [](float x) { return TF32 ? round_tf32(x) : x; };
+  auto lstore = [&](int st) {
+    float* la = lds[st];
+    float* lb = lds[st] + BK * PA;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float x = r[i][2 * e], y = r[i][2 * e + 1];
-      if constexpr (TF32) x = round_tf32(x), y = round_tf32(y);
-      const uint32_t ux = __float_as_uint(x) & 0x7fffffffu, uy = __float_as_uint(y) & 0x7fffffffu;
-      most = max(max(most, ux), uy);
-      least = min(min(least, ux - 1), uy - 1);
+    for (int i = 0; i < CHA; ++i)
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
-        w[p][e] = pack_bf16x2(x, y);
-        if (p + 1 < P) x -= bf16_lo(w[p][e]), y -= bf16_hi(w[p][e]);
+      for (int e = 0; e < 4; ++e) la[(akc[i] + e) * PA + arow[i]] = tf(ra[i][e]);
+#pragma unroll
+    for (int i = 0; i < CHB; ++i) {
+      if constexpr (B_NMAJOR) {
+        *reinterpret_cast<f32x4_t*>(&lb[brow[i] * PB + bkc[i]]) =
+            f32x4_t{tf(rb[i][0]), tf(rb[i][1]), tf(rb[i][2]), tf(rb[i][3])};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lb[(bkc[i] + e) * PB + brow[i]] = tf(rb[i][e]);
       }
     }
-#pragma unroll
-    for (int p = 0; p < P; ++p)
-      *reinterpret_cast<u32x4*>(lds + stage * STAGE + dst[i] + p * (i < CA ? PA : PB)) = w[p];
   };
 
-  f32x4_t acc[FM][FN];
+  f32x16_t acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{};
-  const int fr = lane % 16, fq = lane / 16, chunk = (fq ^ ((fr >> 2) & 3)) * 16;
-  const int aofs = (wm * WM + fr) * 64 + chunk, bofs = P * PA + (wn * WN + fr) * 64 + chunk;
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16_t{};
+  const int fr = lane % 32, fk = lane / 32;
   const int nk = (g.K + BK - 1) / BK;
-#pragma unroll
-  for (int i = 0; i < CA + CB; ++i) gload(i, 0);
-#pragma unroll
-  for (int i = 0; i < CA + CB; ++i) {
-    lstore(i, 0);
-    gload(i, BK);
-  }
+  gload(0);
+  lstore(0);
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
-    const char* st = lds + (kt & 1) * STAGE;
-    bf16x8_t bf[P][FN], af[2][P];
+    const bool more = kt + 1 < nk;
+    if (more) gload((kt + 1) * BK);
+    const float* la = lds[kt & 1];
+    const float* lb = lds[kt & 1] + BK * PA;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      af[0][p] = *reinterpret_cast<const bf16x8_t*>(st + p * PA + aofs);
+    for (int kp = 0; kp < BK / 2; ++kp) {
+      float af[FM], bfv[FN];
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bf[p][j] = *reinterpret_cast<const bf16x8_t*>(st + p * PB + bofs + j * 1024);
-    }
+      for (int i = 0; i < FM; ++i) af[i] = la[(2 * kp + fk) * PA + wm * WM + i * 32 + fr];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      if (i + 1 < FM)
+      for (int j = 0; j < FN; ++j) bfv[j] = lb[(2 * kp + fk) * PB + wn * WN + j * 32 + fr];
 #pragma unroll
-        for (int p = 0; p < P; ++p)
-          af[(i + 1) & 1][p] = *reinterpret_cast<const bf16x8_t*>(st + p * PA + aofs + (i + 1) * 1024);
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int c = i * (CA + CB) / FM; c < (i + 1) * (CA + CB) / FM; ++c) {
-        lstore(c, (kt + 1) & 1);  // the other stage: nobody reads it during this k-tile
-        gload(c, (kt + 2) * BK);
-      }
-      auto multiply = [&](int pb, int pa) {
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[pb][j], af[i & 1][pa], acc[i][j], 0, 0, 0);
-      };
-      if constexpr (!TF32) {  // the smallest products first
-        multiply(0, P - 1);
-        multiply(P - 1, 0);
-      }
-      multiply(1, 1);
-      multiply(0, 1);
-      multiply(1, 0);
-      multiply(0, 0);
-      // two VALU instructions of the split behind each MFMA; the 256-row fp32 tile runs 2-3 % faster in the
-      // compiler's own order (661 against 681 us at 4096^3)
-      if constexpr (TF32 || BM < 256)
-#pragma unroll
-        for (int x = 0; x < FN * (TF32 ? 4 : 6); ++x) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-        }
+        for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bfv[j], af[i], acc[i][j], 0, 0, 0);
+      if (kp == BK / 4 - 1 && more) lstore((kt + 1) & 1);  // the other stage: nobody reads it during this k-tile
     }
     __syncthreads();
   }
-  uint32_t sums = 0;
+  // lane holds C row m0 + wm*WM + i*32 + lane%32, columns n0 + wn*WN + j*32 + 8*q + 4*(lane/32) .. +4
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + wm * WM + i * 32 + fr;
+    if (m >= g.M) continue;
+    float* crow = g.c + int64_t(m) * g.scm;
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sums = max(sums, __float_as_uint(acc[i][j][e]) & 0x7fffffffu);
-  if (__syncthreads_or(sums >= 0x7f800000u || most >= 0x7f7f8000u || least < 0x08800000u - 1)) {
-    // fp32 MFMAs on fragments straight from memory (lane l: row or column l % 16, k = l / 16 of 4)
-    constexpr int U = 4;
-    const float* ap[FM];
-    const float* bp[FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i) ap[i] = g.a + int64_t(min(m0 + wm * WM + i * 16 + fr, g.M - 1)) * g.sam;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) bp[j] = g.b + int64_t(min(n0 + wn * WN + j * 16 + fr, g.N - 1)) * sbn;
-    auto value = [](float x) { return TF32 ? round_tf32(x) : x; };
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{};
-    for (int k0 = 0; k0 < g.K; k0 += 4 * U) {
-      float av[U][FM], bv[U][FN];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = k0 + 4 * u + fq;
-        const bool in = k < g.K;
-#pragma unroll
-        for (int i = 0; i < FM; ++i) av[u][i] = in ? value(ap[i][k]) : 0.0f;
-#pragma unroll
-        for (int j = 0; j < FN; ++j) bv[u][j] = in ? value(bp[j][int64_t(k) * sbk]) : 0.0f;
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + wn * WN + j * 32 + 8 * q + 4 * fk;
+        const f32x4_t v{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        if (n + 4 <= g.N && (reinterpret_cast<uintptr_t>(crow + n) & 15) == 0) {
+          *reinterpret_cast<f32x4_t*>(crow + n) = v;
+        } else {
+          for (int e = 0; e < 4 && n + e < g.N; ++e) crow[n + e] = v[e];
+        }
       }
+  }
+}
+
+// fp32 MFMA GEMM reading its fragments 16 bytes at a time: both operands sit in LDS as k-contiguous rows (A as it
+// lies; a K-contiguous B as it lies, an N-contiguous B transposed while it is staged), row pitch BK + 4 floats (the
+// 16 rows of a quarter-wave's 16-byte reads fall on distinct banks). The k-tile of 32 is taken in 4 groups of 8 k:
+// lane l (row or column l % 32, half h = l / 32) reads k = 8 g + 4 h .. +4 of group g in one ds_read_b128, and MFMA
+// step s of the group uses its element s -- k = 8 g + s for half 0 and 8 g + 4 + s for half 1 -- so 4 MFMA steps
+// take one read per fragment instead of four. (The products are summed in that k order.) The next group's
+// fragments are read while the current group's MFMAs issue; the next k-tile is loaded into registers at the start
+// of a k-tile and stored into the other LDS stage after its second group.
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool B_NMAJOR, bool TF32, bool PF = true>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_mfma_f32q(const F32Args g) {
+  constexpr int NT = 64 * WAVES_M * WAVES_N, BK = 32, P = BK + 4;
+  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 32, FN = WN / 32;
+  constexpr int CHA = BM * BK / 4 / NT, CHB = BN * BK / 4 / NT;  // 16-byte chunks per thread per k-tile
+  static_assert(FM >= 1 && FN >= 1 && CHA >= 1 && CHB >= 1 && CHA * NT * 4 == BM * BK && CHB * NT * 4 == BN * BK,
+                "tile shape");
+  static_assert(!B_NMAJOR || (BN % 32 == 0 && BK % 8 == 0), "N-contiguous B staging");
+  __shared__ __attribute__((aligned(16))) float lds[2][(BM + BN) * P];  // [stage][A rows | B rows]
+  int pid_m, pid_n;
+  tile_coords(blockIdx.x, g.M, g.N, BM, BN, pid_m, pid_n);
+  const int m0 = pid_m * BM, n0 = pid_n * BN;
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+
+  // A (and a K-contiguous B) chunk c: row c / 8, k 4 (c % 8) .. +4. N-contiguous B chunk c: k row kk, columns
+  // 4 nn .. +4 with 8 lanes along n (128 contiguous bytes) and 8 along k
+  const float* asrc[CHA];
+  const float* bsrc[CHB];
+  int adst[CHA], akc[CHA], bdst[CHB], bkc[CHB];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+  for (int i = 0; i < CHA; ++i) {
+    const int c = tid + NT * i, row = c / 8;
+    akc[i] = 4 * (c % 8);
+    asrc[i] = g.a + int64_t(min(m0 + row, g.M - 1)) * g.sam + akc[i];
+    adst[i] = row * P + akc[i];
+  }
+#pragma unroll
+  for (int i = 0; i < CHB; ++i) {
+    const int c = tid + NT * i;
+    if constexpr (B_NMAJOR) {
+      constexpr int NH = BN / 32;  // groups of 8 column chunks
+      const int nn = ((c / 64) % NH) * 8 + c % 8, kk = (c / (64 * NH)) * 8 + (c / 8) % 8;
+      bkc[i] = kk;
+      bsrc[i] = g.b + min(n0 + 4 * nn, g.N - 4);
+      bdst[i] = BM * P + 4 * nn * P + kk;
+    } else {
+      const int row = c / 8;
+      bkc[i] = 4 * (c % 8);
+      bsrc[i] = g.b + int64_t(min(n0 + row, g.N - 1)) * g.sbn + bkc[i];
+      bdst[i] = BM * P + row * P + bkc[i];
+    }
+  }
+  f32x4_t ra[CHA], rb[CHB];
+  auto gload = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < CHA; ++i)
+      ra[i] = (k0 + akc[i] < g.K) ? *reinterpret_cast<const f32x4_t*>(asrc[i] + k0) : f32x4_t{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < CHB; ++i) {
+      if constexpr (B_NMAJOR)
+        rb[i] = (k0 + bkc[i] < g.K) ? *reinterpret_cast<const f32x4_t*>(bsrc[i] + int64_t(k0 + bkc[i]) * g.sbk)
+                                    : f32x4_t{0, 0, 0, 0};
+      else
+        rb[i] = (k0 + bkc[i] < g.K) ? *reinterpret_cast<const f32x4_t*>(bsrc[i] + k0) : f32x4_t{0, 0, 0, 0};
+    }
+  };
+  auto tf = [](float x) { return TF32 ? round_tf32(x) : x; };
+  auto lstore = [&](int st) {
+    float* l = lds[st];
+#pragma unroll
+    for (int i = 0; i < CHA; ++i)
+      *reinterpret_cast<f32x4_t*>(l + adst[i]) = f32x4_t{tf(ra[i][0]), tf(ra[i][1]), tf(ra[i][2]), tf(ra[i][3])};
+#pragma unroll
+    for (int i = 0; i < CHB; ++i) {
+      if constexpr (B_NMAJOR) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) l[bdst[i] + e * P] = tf(rb[i][e]);
+      } else {
+        *reinterpret_cast<f32x4_t*>(l + bdst[i]) = f32x4_t{tf(rb[i][0]), tf(rb[i][1]), tf(rb[i][2]), tf(rb[i][3])};
+      }
+    }
+  };
+
+  f32x16_t acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16_t{};
+  const int fr = lane % 32, fh = lane / 32;
+  const int nk = (g.K + BK - 1) / BK;
+  gload(0);
+  lstore(0);
+  __syncthreads();
+  for (int kt = 0; kt < nk; ++kt) {
+    const bool more = kt + 1 < nk;
+    if (more) gload((kt + 1) * BK);
+    const float* la = lds[kt & 1];
+    const float* lb = lds[kt & 1] + BM * P;
+    f32x4_t af[2][FM], bf[2][FN];  // fragments of group q and q + 1
+    auto frags = [&](int q, int sl) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        af[sl][i] = *reinterpret_cast<const f32x4_t*>(la + (wm * WM + i * 32 + fr) * P + 8 * q + 4 * fh);
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        bf[sl][j] = *reinterpret_cast<const f32x4_t*>(lb + (wn * WN + j * 32 + fr) * P + 8 * q + 4 * fh);
+    };
+    if (PF) frags(0, 0);
+#pragma unroll
+    for (int q = 0; q < BK / 8; ++q) {
+      if (PF && q + 1 < BK / 8) frags(q + 1, (q + 1) & 1);
+      if (!PF) frags(q, q & 1);
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
           for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[u][j], av[u][i], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[q & 1][j][st], af[q & 1][i][st], acc[i][j], 0, 0, 0);
+      if (q == 1 && more) lstore((kt + 1) & 1);  // the other stage: nobody reads it during this k-tile
     }
+    __syncthreads();
   }
-  // lane holds C row m0 + wm*WM + i*16 + lane%16, columns n0 + wn*WN + j*16 + 4*(lane/16) .. +4
+  // lane holds C row m0 + wm*WM + i*32 + lane%32, columns n0 + wn*WN + j*32 + 8*q + 4*(lane/32) .. +4
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
-    const int m = m0 + wm * WM + i * 16 + fr;
+    const int m = m0 + wm * WM + i * 32 + fr;
     if (m >= g.M) continue;
     float* crow = g.c + int64_t(m) * g.scm;
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int n = n0 + wn * WN + j * 16 + 4 * fq;
-      if (n + 4 <= g.N && (reinterpret_cast<uintptr_t>(crow + n) & 15) == 0) {
-        *reinterpret_cast<f32x4_t*>(crow + n) = acc[i][j];
-      } else {
-        for (int e = 0; e < 4 && n + e < g.N; ++e) crow[n + e] = acc[i][j][e];
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + wn * WN + j * 32 + 8 * q + 4 * fh;
+        const f32x4_t v{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        if (n + 4 <= g.N && (reinterpret_cast<uintptr_t>(crow + n) & 15) == 0) {
+          *reinterpret_cast<f32x4_t*>(crow + n) = v;
+        } else {
+          for (int e = 0; e < 4 && n + e < g.N; ++e) crow[n + e] = v[e];
+        }
       }
-    }
   }
 }
 
@@ -1641,25 +1710,22 @@ int launch_mfma_auto(const MfmaArgs& g, hipStream_t s) {
   return launch_mfma_shape<1, false, SILU>(g, s);
 }
 
-// Tile shape by the time of a k-tile on the busiest CU, measured in us: 2.7 per 256x128 tile and 1.85 per 128x128 tile
-// (one block per CU), 0.45 + 0.55 t for t 64x64 tiles (three blocks per CU). 2048^3 176 / 120 / 161 us with the three,
-// 1024^3 89 / 61 / 32, 3000 x 2000 x 3000 257 / 330 / 336, 2500 x 1000 x 520 52 / 36 / 37.
+// 256x256 tiles (16 waves, 16-byte fragment reads) when they fill the CUs at least once, else 128x128 (8 waves).
+// 4096^3 "ieee" with an N-contiguous B: 1051 us with gemm_mfma_f32<256, 256, 4, 4> -> 982 us (torch.matmul 914 us);
+// 128x128 / 256x256 tiles with 4 or 8 waves of 64x64 .. 128x128 measured 1042-1108 us. The tf32 rounding adds
+// registers that the next group's fragments would spill, so that variant reads them as it goes.
 template <bool B_NMAJOR, bool TF32>
 int launch_f32(const F32Args& g, hipStream_t s) {
-  auto tiles = [&](int bm, int bn) { return int64_t((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
-  auto per_cu = [](int64_t t) { return double((t + 255) / 256); };
-  const double big = 2.7 * per_cu(tiles(256, 128)), mid = 1.85 * per_cu(tiles(128, 128)),
-               small = 0.45 + 0.55 * per_cu(tiles(64, 64));
-  if (tiles(64, 64) > INT32_MAX) return invalid("matmul: matrix too large");
-  if (big <= mid && big <= small)
-    hipLaunchKernelGGL((gemm_split_f32<256, 128, 4, 2, B_NMAJOR, TF32>), dim3(unsigned(tiles(256, 128))), dim3(512), 0,
-                       s, g);
-  else if (mid <= small)
-    hipLaunchKernelGGL((gemm_split_f32<128, 128, 4, 2, B_NMAJOR, TF32>), dim3(unsigned(tiles(128, 128))), dim3(512), 0,
-                       s, g);
-  else
-    hipLaunchKernelGGL((gemm_split_f32<64, 64, 2, 2, B_NMAJOR, TF32>), dim3(unsigned(tiles(64, 64))), dim3(256), 0, s,
+  const int64_t big = int64_t((g.M + 255) / 256) * ((g.N + 255) / 256);
+  if (big >= 256) {
+    if (big > INT32_MAX) return invalid("matmul: matrix too large");
+    hipLaunchKernelGGL((gemm_mfma_f32q<256, 256, 4, 4, B_NMAJOR, TF32, !TF32>), dim3(unsigned(big)), dim3(1024), 0, s,
                        g);
+    return check_launch("matmul");
+  }
+  const int64_t tiles = int64_t((g.M + 127) / 128) * ((g.N + 127) / 128);
+  if (tiles > INT32_MAX) return invalid("matmul: matrix too large");
+  hipLaunchKernelGGL((gemm_mfma_f32<128, 128, 2, 4, B_NMAJOR, TF32>), dim3(unsigned(tiles)), dim3(512), 0, s, g);
   return check_launch("matmul");
 }
 

@@ -297,7 +297,7 @@ def test_many_tiles_silu_is_bitwise_two_step(M, N, K):
     assert torch.equal(matmul_silu_and_mul(a, w), silu_and_mul(matmul(a, w.t())))
 
 
-# One shape per tile of gemm_split_f32 (64x64, 128x128, 256x128), cut short in rows, columns and k.
+# fp32 products whose tiles are cut short in rows, columns and k (128x128 tiles).
 F32_SHAPES = [(301, 200, 100), (2044, 2044, 36), (2044, 4092, 44), (67, 68, 4)]
 
 
@@ -326,9 +326,9 @@ def _round_tf32(x):
 @pytest.mark.parametrize("a_scale,b_scale", [(1.0, 1.0), (2.0 ** -107, 2.0 ** 100), (2.0 ** 60, 2.0 ** 55),
                                              (2.0 ** -124, 2.0 ** 100)])
 def test_fp32_parts_keep_fp32_accuracy(M, N, K, nmajor, prec, a_scale, b_scale):
-    """The bf16 parts of fp32 (tf32) inputs give the fp32 product: each of K products and sums rounds at 2^-24 of the
-    running sum, which is at most the product's scale sqrt(K), so the 2-norm of the error stays under sqrt(K) 2^-24 of
-    the result's. At 2^-107 the parts end just above the smallest bf16 denormal, at 2^-124 the fp32 MFMAs take over."""
+    """fp32 (tf32) inputs give the fp32 product also near the ends of the range: each of K products and sums rounds at
+    2^-24 of the running sum, which is at most the product's scale sqrt(K), so the 2-norm of the error stays under
+    sqrt(K) 2^-24 of the result's. (bf16 parts of a value end just above the smallest bf16 denormal at 2^-107.)"""
     a, b = _f32_operands(M, N, K, nmajor, M + K, a_scale, b_scale)
     ref = _f64_product(a, b, prec)
     err = (matmul(a, b, prec).cpu().double() - ref).norm() / ref.norm()
@@ -367,3 +367,31 @@ def test_fused_silu_at_every_finite_gate(M):
     x = torch.eye(64, dtype=torch.bfloat16, device=DEV).repeat(M // 64, 1)
     gate = values.t().repeat(M // 64, 1).to(DEV)
     assert torch.equal(matmul_silu_and_mul(x, w), silu_and_mul(torch.cat([gate, torch.ones_like(gate)], dim=1)))
+
+
+@pytest.mark.parametrize("nmajor", [False, True])
+@pytest.mark.parametrize("prec", ["ieee", "tf32"])
+@pytest.mark.parametrize("n", [100, 512])
+def test_fp32_single_terms_round_once(n, prec, nmajor):
+    """A diagonal A leaves one nonzero term per output: fp32 products that are added in fp32 are then rounded once, to
+    the fp32 value nearest the exact product."""
+    _, b = _f32_operands(1, n, n, nmajor, n)
+    d = torch.randn(n, generator=torch.Generator("cpu").manual_seed(n + 1)).to(DEV)
+    got = matmul(torch.diag(d), b, prec)
+    assert torch.equal(got.cpu(), _f64_product(torch.diag(d), b, prec).float())
+
+
+@pytest.mark.parametrize("M,N,K", F32_SHAPES)
+@pytest.mark.parametrize("prec", ["ieee", "tf32"])
+@pytest.mark.parametrize("value", [math.inf, math.nan, 2.0 ** -120])
+def test_fp32_outputs_do_not_depend_on_other_rows(M, N, K, prec, value):
+    """An unusual value in one row of A and one column of B leaves every other output's bits alone."""
+    a, b = _f32_operands(M, N, K, False, M + K)
+    c = matmul(a, b, prec)
+    a2, b2 = a.clone(), b.t().clone().t()
+    a2[M // 2, 1] = value
+    b2[2, N // 3] = value
+    c2 = matmul(a2, b2, prec)
+    rows = torch.arange(M, device=DEV) != M // 2
+    cols = torch.arange(N, device=DEV) != N // 3
+    assert torch.equal(c[rows][:, cols], c2[rows][:, cols])
