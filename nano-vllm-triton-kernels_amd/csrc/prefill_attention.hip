@@ -613,9 +613,10 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// The prefill attention of one sequence over the paged cache (a prompt chunk and its cached prefix), D = 128, with
-// cache blocks of whole key tiles: the grid, the query tiles, the key splits and the arithmetic of
-// prefill_attention_kernel, for a block of 4 waves in which a wave owns 64 queries.
+// The prefill attention over the paged cache without decode requests (one prompt chunk and its cached prefix, or any
+// sequences of a model with more than 16 q heads per kv head), D = 128, with cache blocks of whole key tiles: the grid, the
+// query tiles, the key splits and the arithmetic of prefill_attention_kernel, for a block of 4 waves in which a wave owns
+// 64 queries.
 //
 // What bounded prefill_attention_kernel here: every K and V fragment that a wave of 32 queries reads from LDS feeds one
 // MFMA (128 bytes per clock and CU, the LDS rate), the K / V tiles pass through registers with per-key row arithmetic,
@@ -1286,16 +1287,19 @@ extern "C" int nvhip_prefill_attention_bf16(void* out, const void* q, const void
                                  dws ? workspace_size - off : 0, s);
     }
   }
+  // prefill_wide_kernel: calls over the paged cache that leave no sequence to the decode attention, with key tiles within
+  // cache blocks. That is one sequence, or several with more than 16 q heads per kv head (64 / 2 heads, 4 x 1024 queries
+  // over 4096 keys 620 -> 503 us; 32 / 1 heads, 32 one-query sequences of 1000 keys and 500 queries over 3000 193 -> 162,
+  // 8 ragged sequences of up to 2000 queries 270 both), in grid order.
+  const bool wide = paged && D == 128 && g.lq_skip == 0 && block_size % kBK == 0 && Hkv < (int64_t(1) << 16);
   // block_plan: lanes for sequences, eighths of the head groups for XCDs. 24 prompts of 30 .. 2100 tokens 259 ->
   // 209-217 us, 48 decode requests and a chunk of 464 queries 87 -> 70, 7 and a chunk of 2000 over 5000 cached keys
   // 486 -> 278 (q/k norm kernel included); the plan takes a block ~0.5 us, and sequences of one length are in its
   // order already (4 x 2048 tokens 81 us without, 83 with it).
   const bool ragged = total_q < num_seqs * max_seqlen_q;
-  g.plan = ragged && num_seqs <= 64 && g.nhg % 8 == 0 && g.splits == 1 && qtiles < 256 ? int(num_seqs) : 0;
+  g.plan = !wide && ragged && num_seqs <= 64 && g.nhg % 8 == 0 && g.splits == 1 && qtiles < 256 ? int(num_seqs) : 0;
   const dim3 grid(static_cast<unsigned>(blocks + g.dec_extra));
 #define NVHIP_PREFILL_LAUNCH(DD, PG, HBV) hipLaunchKernelGGL((prefill_attention_kernel<DD, PG, HBV>), grid, block, 0, s, g)
-  // one sequence over the paged cache (no decode requests in the launch), its key tiles within cache blocks
-  const bool wide = paged && D == 128 && g.lq_skip == 0 && block_size % kBK == 0 && Hkv < (int64_t(1) << 16);
   if (wide && hb == 2) hipLaunchKernelGGL((prefill_wide_kernel<2>), grid, dim3(kWideThreads), 0, s, g);
   else if (wide) hipLaunchKernelGGL((prefill_wide_kernel<1>), grid, dim3(kWideThreads), 0, s, g);
   else if (hb == 2 && D == 64 && paged) NVHIP_PREFILL_LAUNCH(64, true, 2);

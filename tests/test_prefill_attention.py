@@ -412,3 +412,38 @@ def test_infinite_value_of_the_last_key(lq, lk, block_size, causal, Hq, Hkv):
     assert torch.all(got[rows, :, 5] == float("inf")) and torch.all(got[rows, :, 77] == float("-inf"))
     dims = [d for d in range(128) if d not in (5, 77)]
     assert torch.equal(got[:, :, dims], out[:, :, dims])
+
+
+@pytest.mark.parametrize("block_size", [48, 64, 256])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv", [(32, 1), (20, 1), (17, 1)])
+def test_ragged_sequences_of_many_heads_per_kv_head(Hq, Hkv, causal, block_size):
+    """More than 16 q heads per kv head: no sequence is left to the decode attention, so several sequences, one-query and
+    empty ones among them, are query tiles over the cache."""
+    lq, lk = [1, 0, 130, 65, 1, 200], [300, 0, 131, 400, 64, 200]
+    q, kc, vc, bt = paged_case(lq, lk, block_size, Hq=Hq, Hkv=Hkv, seed=Hq + block_size)
+    check(q, kc, vc, cu(lq), cu(lk), causal, bt)
+
+
+@pytest.mark.parametrize("lq", [96, 300])
+def test_graph_replay_over_a_longer_prefix(lq):
+    """One sequence over the cache, captured over a short prefix and replayed over longer ones within the captured
+    max_seqlen_k (query tiles and key splits follow from that one), then over the short one again."""
+    cap, lks = 4096, [lq + 64, 4096, 1500, 3001, lq + 64]
+    q, kc, vc, bt = (x.to(DEV) for x in paged_case([lq], [cap], 256, seed=lq))
+    cq, ck = cu([lq]).to(DEV), cu([lks[0]]).to(DEV)
+
+    def call():
+        return flash_attn_varlen_func(q, kc, vc, lq, cq, cap, ck, 128 ** -0.5, True, bt)
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for lk in lks:
+        ck.copy_(cu([lk]))
+        graph.replay()
+        got = out.clone()
+        assert torch.equal(got, call()), lk
+        ref = oracle.varlen_attention(q.cpu(), kc.cpu(), vc.cpu(), cu([lq]), cu([lk]), 128 ** -0.5, True, bt.cpu())
+        torch.testing.assert_close(got.cpu().float(), ref.float(), rtol=1.6e-2, atol=1e-2)
