@@ -529,8 +529,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_stream_nt(const M
   // No output register: the load's only result is 16 bytes per lane at LDS address dst + 16 lane, which the waits
   // before the barriers below cover.
   auto dma = [&](const u32x4& rsrc, uint32_t vofs, uint32_t dst, int kt) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(vofs),
-                 "s"(rsrc), "s"(uint32_t(kt) * (BK * 2))
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(dst), "v"(vofs), "s"(rsrc),
+                 "s"(uint32_t(kt) * (BK * 2))
                  : "memory");
   };
   auto dma_q = [&](auto qc) {  // load q of a refill

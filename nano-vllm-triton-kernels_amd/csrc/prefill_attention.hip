@@ -726,8 +726,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
   uint64_t k_at = 0, v_at = 0;
   const uint64_t zero_row = reinterpret_cast<uint64_t>(kZeroRow);
   auto dma = [&](uint32_t dst, uint32_t ofs, uint64_t p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(ofs), "s"(p)
-                 : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(dst), "v"(ofs), "s"(p) : "memory");
   };
   // One event's loads: next_load() prepares them, load(0 .. 3) issues V's and load(4 .. 7) K's.
   auto next_load = [&]() {

@@ -1,5 +1,8 @@
 """Host-side behaviour of the Python layer (CPU only): the reference's argument assertions, output shapes through
 the ops' fake (meta) implementations, and no CPU fallback (CPU tensors are refused by the dispatcher)."""
+import pathlib
+import re
+
 import pytest
 import torch
 
@@ -120,3 +123,15 @@ def test_every_op_has_its_native_implementation():
     assert defined == {f"nvhip::{name}" for name in ops._OPS}
     for name in ops._OPS:
         assert torch._C._dispatch_has_kernel_for_dispatch_key(f"nvhip::{name}", "CUDA"), name
+
+
+def test_no_asm_writes_m0_itself():
+    """The compiler keeps values of its own in m0 and cannot be told that an asm statement overwrites it (it is a
+    reserved register in a clobber list): a statement that needs a value there takes it as an operand in m0."""
+    csrc = pathlib.Path(__file__).resolve().parent.parent / "nano-vllm-triton-kernels_amd" / "csrc"
+    operands = 0
+    for path in sorted(csrc.glob("*.hip")) + sorted(csrc.glob("*.h")):
+        for statement in re.findall(r"asm\s+volatile\s*\((.*?)\);", path.read_text(), re.S):
+            assert not re.search(r"\bm0\s*,", statement), (path.name, statement)
+            operands += '"{m0}"' in statement
+    assert operands == 2  # the loads into LDS of gemm_stream_nt and prefill_wide_kernel
