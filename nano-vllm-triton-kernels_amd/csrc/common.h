@@ -84,17 +84,18 @@ __device__ __forceinline__ float round_bf16(float a) { return bf16_lo(pack_bf16x
 __device__ __forceinline__ float silu_bf16(float g) { return round_bf16(g / (1.0f + expf(-g))); }
 
 // silu_bf16 of N bf16 values, the same bits for less: g * rcp(1 + 2^(-g log2 e)) with the hardware exp and reciprocal
-// is within 7 ulps of the formula above for |g| < 8 (3 from rounding g log2 e, 1 each from exp and rcp, 1/2 each from
-// the sum and the product), so its rounding to bf16 is the same unless it lies within 8 ulps of a tie; where one of
-// the N does, or is larger (or NaN), all N take the exact form. 9 VALU instructions instead of about 25 per value (the
-// correctly rounded divide and the exact expf).
+// is within 11 ulps of the formula above for |g| < 8 (the worst over all bf16 g with exp2, rcp and expf each off by up to
+// an ulp; up to 6.4 of them come from rounding g log2 e), so its rounding to bf16 is the same unless it lies within 12
+// ulps of a tie; where one of the N does, or is larger (or NaN), all N take the exact form. No wider: 15 ulps from a tie
+// lie -1.42 and +-0.224, which a wave of gates often holds (16384 tokens' post-attention block 364.5 -> 374.6 us). 9 VALU
+// instructions instead of about 25 per value (the correctly rounded divide and the exact expf).
 template <int N>
 __device__ __forceinline__ void silu_bf16_n(const float (&g)[N], float (&o)[N]) {
   bool exact = false;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     o[i] = g[i] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g[i] * -1.44269504f));
-    exact |= (__float_as_uint(o[i]) & 0xffffu) - 0x7ff8u <= 16u || !(__builtin_fabsf(g[i]) < 8.0f);
+    exact |= (__float_as_uint(o[i]) & 0xffffu) - 0x7ff4u <= 24u || !(__builtin_fabsf(g[i]) < 8.0f);
   }
   if (exact) {
 #pragma unroll

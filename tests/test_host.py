@@ -3,6 +3,7 @@ the ops' fake (meta) implementations, and no CPU fallback (CPU tensors are refus
 import pathlib
 import re
 
+import numpy as np
 import pytest
 import torch
 
@@ -135,3 +136,25 @@ def test_no_asm_writes_m0_itself():
             assert not re.search(r"\bm0\s*,", statement), (path.name, statement)
             operands += '"{m0}"' in statement
     assert operands == 2  # the loads into LDS of gemm_stream_nt and prefill_wide_kernel
+
+
+def test_fast_silu_window_holds_its_error():
+    """silu_bf16_n takes the exact form where its fast one is near a bf16 tie: the window has to hold the largest
+    distance of the two over all bf16 gates below 8, the hardware exp and reciprocal and expf each off by up to an ulp."""
+    common = pathlib.Path(__file__).resolve().parent.parent / "nano-vllm-triton-kernels_amd" / "csrc" / "common.h"
+    low, width = (int(x, 0) for x in re.search(r"& 0xffffu\) - (\w+)u <= (\w+)u", common.read_text()).groups())
+    window = min(0x8000 - low, low + width - 0x8000)
+    f32 = np.float32
+    g = (np.arange(65536, dtype=np.uint32) << 16).view(f32)
+    g = g[np.abs(g) < 8]
+    bits = lambda x: x.astype(f32).view(np.int32).astype(np.int64)
+    off = lambda x, ulps: (bits(x) + ulps).astype(np.int32).view(f32)
+    t = (g * f32(-1.44269504)).astype(f32)
+    exact = [bits(g / (f32(1) + off(np.exp(-g.astype(np.float64)), a))) for a in (-1, 0, 1)]
+    worst = 0
+    for a in (-1, 0, 1):
+        rcp = 1 / (f32(1) + off(np.exp2(t.astype(np.float64)), a)).astype(np.float64)
+        for b in (-1, 0, 1):
+            fast = bits(g * off(rcp, b))
+            worst = max(worst, *(int(np.abs(fast - x).max()) for x in exact))
+    assert 6 < worst <= window, (worst, window)

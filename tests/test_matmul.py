@@ -358,10 +358,14 @@ def test_fp32_values_without_parts(M, N, K, nmajor, prec):
 
 
 @pytest.mark.parametrize("M", [256, 2304])   # the staged and the streaming kernel's epilogue
-def test_fused_silu_at_every_finite_gate(M):
+@pytest.mark.parametrize("adjacent", [False, True])
+def test_fused_silu_at_every_finite_gate(M, adjacent):
     """One-hot rows of x pick single weights, so the gates are every finite bf16 value: the fused epilogue's silu is
-    bitwise the unfused kernel's (torch's formula with the exact exp and divide)."""
-    values = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(1024, 64).clone()
+    bitwise the unfused kernel's (torch's formula with the exact exp and divide). adjacent: neighbouring columns hold
+    neighbouring bit patterns, so that the values which an epilogue takes together are all below 8 or all above it (64
+    patterns apart, each of 2 .. 8 stands with one that sends its group to the exact form)."""
+    values = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    values = (values.view(64, 1024).t() if adjacent else values.view(1024, 64)).clone()
     values[~values.isfinite()] = 0.0
     w = torch.cat([values, torch.ones_like(values)]).to(DEV)
     x = torch.eye(64, dtype=torch.bfloat16, device=DEV).repeat(M // 64, 1)
