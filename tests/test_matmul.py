@@ -11,6 +11,8 @@ shape M selects, fp32 4096^3, strided/offset views and the committed golden prod
 """
 import math
 import os
+import pathlib
+import re
 
 import numpy as np
 import pytest
@@ -295,6 +297,54 @@ def test_many_tiles_silu_is_bitwise_two_step(M, N, K):
     a = (torch.randn(M, K, generator=g) / math.sqrt(K)).to(torch.bfloat16).to(DEV)
     w = torch.randn(2 * inter, K, generator=g).to(torch.bfloat16).to(DEV)
     assert torch.equal(matmul_silu_and_mul(a, w), silu_and_mul(matmul(a, w.t())))
+
+
+# ... and more tiles than blocks, so that a block goes on to a second tile (and a third where the count passes 512): the
+# tile that launch_stream_shape picks, then M, N, K. One to 48 k-tiles per tile, so that the loads run up to several
+# tiles ahead; tile counts that the eight XCDs do not share evenly.
+STREAM_ROUNDS = [
+    (256, 256, 1545, 23312, 64), (256, 256, 1027, 21840, 128), (256, 256, 2315, 16448, 192),
+    (256, 256, 1039, 21776, 1024), (256, 192, 1347, 21792, 64), (256, 192, 651, 21936, 128),
+    (256, 192, 1413, 21888, 192), (256, 192, 1157, 14656, 1024), (192, 256, 1293, 21840, 64),
+    (192, 256, 901, 16432, 128), (192, 256, 1285, 21936, 192), (192, 256, 771, 21168, 1024),
+    (256, 128, 2123, 10800, 64), (256, 128, 1283, 10816, 128), (256, 128, 2113, 10784, 192),
+    (256, 128, 1437, 10880, 1024), (128, 256, 1357, 16496, 64), (128, 256, 513, 22208, 128),
+    (128, 256, 1537, 14352, 192), (128, 256, 517, 22208, 1024), (128, 192, 779, 18704, 64),
+    (128, 192, 579, 16496, 128), (128, 192, 645, 21824, 192), (128, 192, 591, 16576, 1024),
+    (192, 128, 1029, 10784, 3072)]
+
+
+def _stream_tiles(M, N, K):
+    """Tile shape and number of tiles by launch_stream_shape's rule, its table read from the source."""
+    source = (pathlib.Path(__file__).resolve().parent.parent / "nano-vllm-triton-kernels_amd" / "csrc" /
+              "gemm.hip").read_text()
+    rule = source[source.index("int launch_stream_shape"):]
+    table = re.search(r"constexpr Shape shapes\[\] = \{(.*?)\}\};", rule, re.S).group(1)
+    shapes = [tuple(map(float, m)) for m in re.findall(r"\{(\d+), (\d+), ([\d.]+), ([\d.]+)", table)]
+    assert len(shapes) == 7
+    costs = []
+    for bm, bn, per_ktile, fixed in shapes:
+        tiles = -(-M // int(bm)) * -(-N // int(bn))
+        full, rest = divmod(tiles, 256)
+        rounds = full + (0.5 + 0.5 * rest / 256 if rest else 0)
+        costs.append((rounds * (K // 64 * per_ktile + fixed), int(bm), int(bn), tiles))
+    return min(costs, key=lambda x: x[0])[1:]
+
+
+@pytest.mark.parametrize("bm,bn,M,N,K", STREAM_ROUNDS)
+def test_more_tiles_than_blocks_are_bitwise_the_staged_kernel(bm, bn, M, N, K):
+    shape_m, shape_n, tiles = _stream_tiles(M, N, K)
+    assert (shape_m, shape_n) == (bm, bn) and tiles > 256 and tiles % 8 != 0
+    g = torch.Generator(DEV).manual_seed(M + N + K)
+    a = (torch.randn(M, K + 24, generator=g, device=DEV) / math.sqrt(K)).to(torch.bfloat16)[:, :K]
+    w = torch.randn(N, K + 8, generator=g, device=DEV).to(torch.bfloat16)[:, :K]
+    c = matmul(a, w.t())
+    assert torch.equal(c, matmul(a, w.t().contiguous()))   # the N-contiguous layout runs gemm_mfma_nt
+    assert torch.equal(matmul_silu_and_mul(a, w), silu_and_mul(c))
+    rows = torch.tensor([0, M // 2, M - 1])
+    cols = torch.tensor([0, 1, N // 2, N - 2, N - 1])
+    ref = oracle.matmul_fp64(a.cpu()[rows], w.cpu()[cols].t())
+    torch.testing.assert_close(c.cpu()[rows][:, cols].double(), ref, rtol=1.6e-2, atol=1e-2)
 
 
 # fp32 products whose tiles are cut short in rows, columns and k (128x128 tiles).
