@@ -5,6 +5,8 @@
 #include <stdint.h>
 
 #include <string>
+#include <type_traits>
+#include <utility>
 
 #include "nvhip.h"
 
@@ -62,6 +64,16 @@ int add_rms_norm_partials(uint16_t* y, uint16_t* res_out, const float* xp, int s
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>): a loop whose counter is a constant in the body.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
 
 // bf16 bits -> fp32 (exact).
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }

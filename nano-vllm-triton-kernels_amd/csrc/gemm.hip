@@ -15,7 +15,6 @@
 //   gemm_mfma_f32  fp32, A K-contiguous, B K- or N-contiguous: 32x32x2 fp32 MFMA (exact products, fp32 sums).
 //   gemm_generic   any dtype/strides/precision: 64x64 tile, 4x4 outputs per thread, fp32 FMA.
 #include <type_traits>
-#include <utility>
 
 #include "common.h"
 
@@ -437,15 +436,6 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_nt(const Mfm
 //
 // Tile order: XCD x takes an eighth of the tiles, in the order of the GROUP_M swizzle, so that its blocks share their
 // operand rows in its L2.
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 constexpr int kStreamBlocks = 256;  // one persistent block per CU
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int NSA, int NSB, bool SILU>

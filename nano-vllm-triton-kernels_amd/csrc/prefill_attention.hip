@@ -32,8 +32,6 @@
 // each (query tile, sequence, head group) is cut into key ranges run by separate blocks; each writes its queries'
 // (max, sum, O) records and prefill_combine merges them in split order.
 #include <algorithm>
-#include <type_traits>
-#include <utility>
 
 #include "decode_attention.h"
 
@@ -602,15 +600,6 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
       *reinterpret_cast<u32x2*>(op + 32 * t + 8 * rr) =
           u32x2{pack_bf16x2(o[t][4 * rr] * inv, o[t][4 * rr + 1] * inv),
                   pack_bf16x2(o[t][4 * rr + 2] * inv, o[t][4 * rr + 3] * inv)};
-}
-
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 // The prefill attention over the paged cache without decode requests (one prompt chunk and its cached prefix, or any
