@@ -20,8 +20,7 @@ byte count; the same kernel at T = 1, 32, 2048, and at T = 2048 with write_k (th
 reference's README table; at T = 2048 enough sets rotate -- 32 -- that the reads come from HBM, as for the headline); the unfused KV write (store_kvcache, bytes =
 T * (2 * 2048 read + 2 * 2048 written + 4 slot)) at T = 8192; RMSNorm, Add+RMSNorm and SiLU x Mul at T = 8192
 (hidden 1024, gate_up 2 x 3072) in GB/s; the bf16 GEMM at the Qwen3-0.6B projection shapes, M = 2048 in TFLOP/s
-and M = 32 in GB/s (weights rotated through >= 512 MiB of copies so they come from HBM); the fp32 4096^3 GEMM
-(its products run as six bf16 products on the matrix cores, so its fraction of the fp32 peak can exceed 1);
+and M = 32 in GB/s (weights rotated through >= 512 MiB of copies so they come from HBM); the fp32 4096^3 GEMM;
 the paged decode attention of one layer for 32 sequences with contexts of 512..2048 tokens, in GB/s; the causal
 prefill attention of one layer over 4 sequences of 2048 tokens and of a 256-token chunk over 3840 cached keys, in
 TFLOP/s; the end-to-end decode step of a

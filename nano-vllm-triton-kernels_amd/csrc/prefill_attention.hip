@@ -603,9 +603,9 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
 }
 
 // The prefill attention over the paged cache without decode requests (one prompt chunk and its cached prefix, or any
-// sequences of a model with more than 16 q heads per kv head), D = 128, with cache blocks of whole key tiles: the grid, the
-// query tiles, the key splits and the arithmetic of prefill_attention_kernel, for a block of 4 waves in which a wave owns
-// 64 queries.
+// sequences of a model with more than 16 q heads per kv head), D = 128, with cache blocks of whole key tiles: the grid,
+// the query tiles, the key splits and the arithmetic of prefill_attention_kernel, for a block of 4 waves in which a wave
+// owns 64 queries.
 //
 // What bounded prefill_attention_kernel here: every K and V fragment that a wave of 32 queries reads from LDS feeds one
 // MFMA (128 bytes per clock and CU, the LDS rate), the K / V tiles pass through registers with per-key row arithmetic,
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
 // The matrix instructions are inline asm, because the compiler's own choice keeps all results in accumulation registers
 // and moves the scores back and forth. It does not know their timing, so nothing may read a result, or write an operand
 // with a vector instruction, right before or after one: every such pair below lies several MFMAs apart, or behind the
-// s_nop fences.
+// s_nop fences, and the build measures the distances in the assembly (check_asm.py).
 // 2048 queries over 14001 cached keys (16 / 8 heads): 326 -> 258-268 us with the q/k norm kernel, 0.77 -> 0.96 PFLOP/s;
 // 256 over 3840 38.5 -> 37. On contiguous keys it was no faster than prefill_attention_kernel (8192 tokens 257-261 us
 // against 266, 16 x 256 tokens 19.5 against 16.6), which keeps those.
@@ -780,8 +780,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
   };
   using Scores = f32x16_t[2][2];  // [u][qh]
   // Masks the scores of the tile at kt0 where it needs it, in front of the barrier that hands out its V rows (slot; one
-  // event's loads were issued after them). Behind the last key those are copies of its row, and 0 times an infinity there
-  // would be NaN: each wave zeroes what it loaded itself.
+  // event's loads were issued after them). Behind the last key those are copies of its row, and 0 times an infinity
+  // there would be NaN: each wave zeroes what it loaded itself.
   auto mask = [&](Scores& s, int kt0, int slot) {
     if (kt0 + kBK <= lk && (!g.causal || kt0 + kBK - 1 <= diag + wave_q0)) return;
     if (kt0 + kBK > lk) {
@@ -1275,10 +1275,10 @@ extern "C" int nvhip_prefill_attention_bf16(void* out, const void* q, const void
                                  dws ? workspace_size - off : 0, s);
     }
   }
-  // prefill_wide_kernel: calls over the paged cache that leave no sequence to the decode attention, with key tiles within
-  // cache blocks. That is one sequence, or several with more than 16 q heads per kv head (64 / 2 heads, 4 x 1024 queries
-  // over 4096 keys 620 -> 503 us; 32 / 1 heads, 32 one-query sequences of 1000 keys and 500 queries over 3000 193 -> 162,
-  // 8 ragged sequences of up to 2000 queries 270 both), in grid order.
+  // prefill_wide_kernel: calls over the paged cache that leave no sequence to the decode attention, with key tiles
+  // within cache blocks. That is one sequence, or several with more than 16 q heads per kv head (64 / 2 heads, 4 x 1024
+  // queries over 4096 keys 620 -> 503 us; 32 / 1 heads, 32 one-query sequences of 1000 keys and 500 queries over 3000
+  // 193 -> 162, 8 ragged sequences of up to 2000 queries 270 both), in grid order.
   const bool wide = paged && D == 128 && g.lq_skip == 0 && block_size % kBK == 0 && Hkv < (int64_t(1) << 16);
   // block_plan: lanes for sequences, eighths of the head groups for XCDs. 24 prompts of 30 .. 2100 tokens 259 ->
   // 209-217 us, 48 decode requests and a chunk of 464 queries 87 -> 70, 7 and a chunk of 2000 over 5000 cached keys
