@@ -784,14 +784,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
   // there would be NaN: each wave zeroes what it loaded itself.
   auto mask = [&](Scores& s, int kt0, int slot) {
     if (kt0 + kBK <= lk && (!g.causal || kt0 + kBK - 1 <= diag + wave_q0)) return;
-    if (kt0 + kBK > lk) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (4 * (bwave + 4 * j) + lr >= lk - kt0)
-          *reinterpret_cast<u32x4*>(lds + (NK + slot) * TILE + j * 4096 + bwave * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
+    if (kt0 > last) return;  // the last tile loaded again, unused
 #pragma unroll
     for (int qh = 0; qh < 2; ++qh) {
       const int lim = min(lk - 1, g.causal ? diag + wave_q0 + 32 * qh + ql : lk - 1) - kt0 - 4 * hf;
@@ -800,6 +793,14 @@ __global__ __launch_bounds__(kWideThreads, 1) void prefill_wide_kernel(const Pre
 #pragma unroll
         for (int r = 0; r < 16; ++r)
           if (32 * u + 8 * (r / 4) + r % 4 > lim) s[u][qh][r] = -INFINITY;
+    }
+    if (kt0 + kBK > lk) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * (bwave + 4 * j) + lr >= lk - kt0)
+          *reinterpret_cast<u32x4*>(lds + (NK + slot) * TILE + j * 4096 + bwave * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   };
   auto max_step = [&](const Scores& s, auto kc) {  // step k of 32: two scores of a query half
