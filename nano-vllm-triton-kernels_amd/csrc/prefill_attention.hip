@@ -1277,10 +1277,13 @@ extern "C" int nvhip_prefill_attention_bf16(void* out, const void* q, const void
     }
   }
   // prefill_wide_kernel: calls over the paged cache that leave no sequence to the decode attention, with key tiles
-  // within cache blocks. That is one sequence, or several with more than 16 q heads per kv head (64 / 2 heads, 4 x 1024
-  // queries over 4096 keys 620 -> 503 us; 32 / 1 heads, 32 one-query sequences of 1000 keys and 500 queries over 3000
-  // 193 -> 162, 8 ragged sequences of up to 2000 queries 270 both), in grid order.
-  const bool wide = paged && D == 128 && g.lq_skip == 0 && block_size % kBK == 0 && Hkv < (int64_t(1) << 16);
+  // within cache blocks and enough of them per block. That is one sequence, or several with more than 16 q heads per kv
+  // head (32 / 1 heads, us: 4 sequences of 30 .. 900 queries over up to 4000 keys 152 -> 105, 32 one-query sequences of
+  // 1000 keys and 500 queries over 3000 189 -> 137), in grid order. Its start costs more: with two heads per block 17
+  // queries over 17 keys took 9.0 us against 8.4, 64 over 64 10.3 against 10.4, 128 over 128 13.2 against 14.1; with one
+  // (twice the queries) 128 over 128 12.2 against 12.3, 130 over 200 16.4 against 16.1, 256 over 256 17.3 against 19.1.
+  const bool wide = paged && D == 128 && g.lq_skip == 0 && block_size % kBK == 0 && Hkv < (int64_t(1) << 16) &&
+                    g.split_len >= 4 * kBK / hb;
   // block_plan: lanes for sequences, eighths of the head groups for XCDs. 24 prompts of 30 .. 2100 tokens 259 ->
   // 209-217 us, 48 decode requests and a chunk of 464 queries 87 -> 70, 7 and a chunk of 2000 over 5000 cached keys
   // 486 -> 278 (q/k norm kernel included); the plan takes a block ~0.5 us, and sequences of one length are in its

@@ -406,8 +406,8 @@ def test_infinite_value_of_the_last_key(lq, lk, block_size, causal, Hq, Hkv):
     out, _ = check(q, kc, vc, cu([lq]), cu([lk]), causal, bt)
     blk, slot = bt[0, (lk - 1) // block_size].long(), (lk - 1) % block_size
     vc[blk, slot, :, 5], vc[blk, slot, :, 77] = float("inf"), float("-inf")
-    got = flash_attn_varlen_func(q.to(DEV), kc.to(DEV), vc.to(DEV), lq, cu([lq]).to(DEV), lk, cu([lk]).to(DEV),
-                                 128 ** -0.5, causal, bt.to(DEV)).cpu()
+    got = flash_attn_varlen_func(q.to(DEV), kc.to(DEV), vc.to(DEV), lq, cu([lq]).to(DEV), max(lk, 256),
+                                 cu([lk]).to(DEV), 128 ** -0.5, causal, bt.to(DEV)).cpu()
     rows = slice(lq - 1, lq) if causal else slice(0, lq)
     assert torch.all(got[rows, :, 5] == float("inf")) and torch.all(got[rows, :, 77] == float("-inf"))
     dims = [d for d in range(128) if d not in (5, 77)]
@@ -447,3 +447,19 @@ def test_graph_replay_over_a_longer_prefix(lq):
         assert torch.equal(got, call()), lk
         ref = oracle.varlen_attention(q.cpu(), kc.cpu(), vc.cpu(), cu([lq]), cu([lk]), 128 ** -0.5, True, bt.cpu())
         torch.testing.assert_close(got.cpu().float(), ref.float(), rtol=1.6e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(16, 8), (4, 4)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("lq,lk", [(17, 17), (33, 1), (64, 64), (65, 65), (100, 127), (128, 128), (130, 255)])
+def test_one_sequence_around_the_kernels_border(lq, lk, causal, Hq, Hkv):
+    """max_seqlen_k picks the kernel (128 keys with two heads per block, 256 with one), whatever the sequence's own length:
+    both give the same bits, also for fewer key tiles than the border says."""
+    q, kc, vc, bt = paged_case([lq], [lk], 64, Hq=Hq, Hkv=Hkv, seed=lq + lk)
+    out, _ = check(q, kc, vc, cu([lq]), cu([lk]), causal, bt)
+    args = [x.to(DEV) for x in (q, kc, vc, cu([lq]), cu([lk]), bt)]
+    for max_k in (lk, 127, 128, 255, 256, 511):
+        if max_k >= lk:
+            got = flash_attn_varlen_func(args[0], args[1], args[2], lq, args[3], max_k, args[4], 128 ** -0.5, causal,
+                                         args[5])
+            assert torch.equal(got.cpu(), out), max_k
