@@ -147,8 +147,9 @@ __device__ __forceinline__ bool block_plan(const PrefillArgs& g, int item, Plan&
   return true;
 }
 
-// HB q heads of one kv head per block (4 waves each, sharing the K/V tiles in LDS).
-template <int D, bool PAGED, int HB>
+// HB q heads of one kv head per block (4 waves each, sharing the K/V tiles in LDS). PLAN: the blocks find their tile with
+// block_plan (its own instance: the code of both in one kernel cost small calls without it 0.3-0.5 us).
+template <int D, bool PAGED, int HB, bool PLAN>
 __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const PrefillArgs g) {
   constexpr int kBQ = block_queries(HB), kHeadThreads = kThreads / HB;
   constexpr int DC = D / 16;   // 16-wide dim steps of Q.K
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
     return;
   }
   int b, hg, qt, split, q0s, lq, k0s, lk;
-  if (g.plan) {  // (no key splits; the head groups divide evenly over the XCDs)
+  if constexpr (PLAN) {  // (no key splits; the head groups divide evenly over the XCDs)
     const int sub = g.nhg / 8, r = blockIdx.x / 8;
     Plan p;
     if (!block_plan<kBQ>(g, r / sub, p)) return;
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
   if (lq >= 1 && lq <= g.lq_skip) {  // the paged decode attention takes this sequence (the whole block: b is uniform)
     // one block per (sequence, kv head) runs the decode attention of the pair (the whole block: b, hg, qt uniform)
     if constexpr (PAGED) {
-      if (g.dec_inline && (g.plan || qt == g.qtiles - 1) && split == 0 && (hg * HB) % g.G == 0) {
+      if (g.dec_inline && (PLAN || qt == g.qtiles - 1) && split == 0 && (hg * HB) % g.G == 0) {
         const int pair = b * g.Hkv + hg * HB / g.G, bid = g.dec.halves ? 2 * pair : pair;
         if (g.dec.bs % 32 == 0) decode_block<D, 16, true, false, true>(g.dec, bid, reinterpret_cast<unsigned char*>(lds));
         else decode_block<D, 16, false, false, true>(g.dec, bid, reinterpret_cast<unsigned char*>(lds));
@@ -623,9 +624,10 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
 // and moves the scores back and forth. It does not know their timing, so nothing may read a result, or write an operand
 // with a vector instruction, right before or after one: every such pair below lies several MFMAs apart, or behind the
 // s_nop fences, and the build measures the distances in the assembly (check_asm.py).
-// 2048 queries over 14001 cached keys (16 / 8 heads): 326 -> 258-268 us with the q/k norm kernel, 0.77 -> 0.96 PFLOP/s;
-// 256 over 3840 38.5 -> 37. On contiguous keys it was no faster than prefill_attention_kernel (8192 tokens 257-261 us
-// against 266, 16 x 256 tokens 19.5 against 16.6), which keeps those.
+// 2048 queries over 14001 cached keys (16 / 8 heads): 326 -> 249 us with the q/k norm kernel, 0.77 -> 1.0 PFLOP/s (262
+// while mask() kept its scalars across the wait: 118 of them spilled); 300 over 4000 39.5 -> 34.2. A form of it for
+// contiguous keys, before that, was no faster than prefill_attention_kernel (8192 tokens 257-261 us against 266, 16 x 256
+// tokens 19.5 against 16.6), which keeps those.
 __device__ const uint32_t kZeroRow[64] = {};  // what the keys of an invalid cache block read
 
 constexpr int kWideThreads = 256;
@@ -1286,12 +1288,21 @@ extern "C" int nvhip_prefill_attention_bf16(void* out, const void* q, const void
                     g.split_len >= 4 * kBK / hb;
   // block_plan: lanes for sequences, eighths of the head groups for XCDs. 24 prompts of 30 .. 2100 tokens 259 ->
   // 209-217 us, 48 decode requests and a chunk of 464 queries 87 -> 70, 7 and a chunk of 2000 over 5000 cached keys
-  // 486 -> 278 (q/k norm kernel included); the plan takes a block ~0.5 us, and sequences of one length are in its
-  // order already (4 x 2048 tokens 81 us without, 83 with it).
-  const bool ragged = total_q < num_seqs * max_seqlen_q;
-  g.plan = !wide && ragged && num_seqs <= 64 && g.nhg % 8 == 0 && g.splits == 1 && qtiles < 256 ? int(num_seqs) : 0;
+  // 486 -> 278 (q/k norm kernel included). It costs a block ~0.5 us and gives nothing where all blocks start at once (a
+  // grid of at most one block per CU: 5 prompts of up to 300 tokens 13.8 us without, 14.4 with it) or where the
+  // sequences are in its order already (of one length, or nearly: 64 of 1000 .. 1100 tokens 463 without, 476 with it, 8
+  // of 500 .. 520 23.4 and 24.5). Of 154 other calls it made 28 slower by 1 .. 6 %, by the luck of the grid order, and
+  // 85 faster by 2 .. 71 %.
+  const bool ragged = double(total_q) < 0.9 * double(num_seqs) * double(max_seqlen_q);
+  g.plan = !wide && ragged && num_seqs <= 64 && g.nhg % 8 == 0 && g.splits == 1 && base_blocks > 256 && qtiles < 256
+               ? int(num_seqs)
+               : 0;
   const dim3 grid(static_cast<unsigned>(blocks + g.dec_extra));
-#define NVHIP_PREFILL_LAUNCH(DD, PG, HBV) hipLaunchKernelGGL((prefill_attention_kernel<DD, PG, HBV>), grid, block, 0, s, g)
+#define NVHIP_PREFILL_LAUNCH(DD, PG, HBV)                                                                      \
+  do {                                                                                                         \
+    if (g.plan) hipLaunchKernelGGL((prefill_attention_kernel<DD, PG, HBV, true>), grid, block, 0, s, g);       \
+    else hipLaunchKernelGGL((prefill_attention_kernel<DD, PG, HBV, false>), grid, block, 0, s, g);             \
+  } while (0)
   if (wide && hb == 2) hipLaunchKernelGGL((prefill_wide_kernel<2>), grid, dim3(kWideThreads), 0, s, g);
   else if (wide) hipLaunchKernelGGL((prefill_wide_kernel<1>), grid, dim3(kWideThreads), 0, s, g);
   else if (hb == 2 && D == 64 && paged) NVHIP_PREFILL_LAUNCH(64, true, 2);

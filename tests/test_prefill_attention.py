@@ -336,9 +336,11 @@ def test_graph_replay_matches_eager():
 @pytest.mark.parametrize("Hq,Hkv,D", [(16, 8, 128), (32, 8, 128), (16, 8, 64)])
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("lq", [
-    [1, 300], [64, 65, 63, 0, 129, 1], [0, 0, 200, 1, 1, 17, 0], [20] * 63 + [321], [1, 2, 8, 9] * 15 + [257, 0, 0, 128]])
+    [1, 300], [64, 65, 63, 0, 129, 1], [0, 0, 200, 1, 1, 17, 0], [20] * 63 + [321], [1, 2, 8, 9] * 15 + [257, 0, 0, 128],
+    [64, 65, 63, 0, 129, 1] * 6, [0, 0, 200, 1, 1, 17, 0] * 4, [700] + [90] * 6, [300] * 40 + [385]])
 def test_ragged_batches_in_plan_order(lq, paged, Hq, Hkv, D):
-    """Up to 64 sequences of different lengths: the blocks find their tiles from the sequence bounds. Empty sequences
+    """Up to 64 sequences of different lengths: with more blocks than CUs and a tenth of the query slots empty, the blocks
+    find their tiles from the sequence bounds (the short lists and the last one stay in grid order). Empty sequences
     first, last and between, tiles cut short, decode requests and short runs behind the long sequences (the cache), a
     full wave of sequences. With empty sequences added until there are more than 64 the blocks take them in grid order:
     every query of the prefill kernel has the same bits."""
