@@ -11,7 +11,7 @@
 // row; without one, one block per row. At 32 x 151936 (a decode step of Qwen3-0.6B) the split form takes 5.8 us and
 // the merge 4; torch's bf16 -> fp32 copy and ArgMaxOps took 6.6 + 59.8 us.
 #include <algorithm>
-#include <cfloat>
+#include <cmath>
 
 #include "common.h"
 
@@ -42,10 +42,12 @@ __device__ __forceinline__ void merge(Best& b, float v, int64_t i) {
 }
 
 // Best of elements [lo, hi) of a row (lo a multiple of 8 when VEC), over the block; the result in thread 0. Whole
-// 16-byte chunks are compared by their maximum: a thread keeps the first chunk whose maximum is the largest and whether
-// it saw a NaN, ~3 VALU instructions per logit instead of ~7 for a (value, 64-bit index) pair per logit, and looks up
-// the element in that chunk at the end; a thread that saw a NaN goes over its chunks again in the full order. 250 x
-// 151936 (76 MB) 21.5 -> 15.5 us, 32 x 151936 6.6 -> 5.8 us.
+// 16-byte chunks are compared by their maximum: a thread keeps the first chunk whose maximum is the largest, ~3 VALU
+// instructions per logit instead of ~7 for a (value, 64-bit index) pair per logit, and looks up the element in that chunk
+// at the end. Of NaNs it keeps the first group of U chunks that holds one (the first chunk itself costs 3 % at 100 x
+// 151936) and looks the first one up there. 250 x 151936 (76 MB) 21.5 -> 15.5 us, 32 x 151936 6.6 -> 5.8 us, with a NaN
+// in every row the same (30.2 us for both launches at 250 rows when a thread that saw one went over its chunks again, 17.7
+// now).
 template <bool VEC>
 __device__ __forceinline__ Best block_best(const uint16_t* row, int64_t lo, int64_t hi) {
   const int tid = threadIdx.x;
@@ -56,42 +58,55 @@ __device__ __forceinline__ Best block_best(const uint16_t* row, int64_t lo, int6
     const u32x4* rv = reinterpret_cast<const u32x4*>(row) + c0;
     const int n = int(c1 - c0);  // of this slice
     constexpr int U = 8;
-    int best = -1;
-    bool nan = false;
+    int best = -1, first_nan = -1;  // chunks; with a NaN: the first of the group of U that holds it, or the chunk itself
+    auto has_nan = [](const float (&f)[8]) {
+      bool nan = false;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) nan |= __builtin_isunordered(f[e], f[e + 1]);
+      return nan;
+    };
     auto take = [&](const u32x4& q, int c) {
       float f[8];
       unpack8(q, f);
       float m = f[0];
 #pragma unroll
       for (int e = 1; e < 8; ++e) m = fmaxf(m, f[e]);
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) nan |= __builtin_isunordered(f[e], f[e + 1]);
       if (m > b.v) b.v = m, best = c;
+      return has_nan(f);
     };
     int c = tid;
+    u32x4 q[U];
     for (; c + (U - 1) * kThreads < n; c += U * kThreads) {
-      u32x4 q[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) q[u] = rv[c + u * kThreads];
+      bool nan = false;
 #pragma unroll
-      for (int u = 0; u < U; ++u) take(q[u], c + u * kThreads);
+      for (int u = 0; u < U; ++u) nan |= take(q[u], c + u * kThreads);
+      if (nan && first_nan < 0) first_nan = c;
     }
-    for (; c < n; c += kThreads) take(rv[c], c);
-    if (nan) {
-      b = Best{-INFINITY, INT64_MAX};
-      for (c = tid; c < n; c += kThreads) {
-        float f[8];
-        unpack8(rv[c], f);
+    const int grouped = c;
+    for (; c < n; c += kThreads)
+      if (take(rv[c], c) && first_nan < 0) first_nan = c;
+    if (first_nan >= 0) {
+      best = first_nan, b.v = NAN;
+      if (first_nan < grouped) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) take_later(b, f[e], (c0 + c) * 8 + e);
+        for (int u = 0; u < U; ++u) q[u] = rv[first_nan + u * kThreads];
+#pragma unroll
+        for (int u = U - 1; u >= 0; --u) {
+          float f[8];
+          unpack8(q[u], f);
+          if (has_nan(f)) best = first_nan + u * kThreads;
+        }
       }
-    } else if (best >= 0) {
+    }
+    if (best >= 0) {
       float f[8];
       unpack8(rv[best], f);
       int at = 7;
 #pragma unroll
       for (int e = 6; e >= 0; --e)
-        if (f[e] == b.v) at = e;
+        if (f[e] == b.v || (first_nan >= 0 && f[e] != f[e])) at = e;
       b.i = (c0 + best) * 8 + at;
     }
     tail = c1 * 8;

@@ -56,6 +56,24 @@ def test_nan_counts_as_the_largest():
     assert got[:5].tolist() == [77, 151935, 3999, 13, 100]
 
 
+@pytest.mark.parametrize("n", [40, 4099, 20000, V])
+def test_several_nans_go_to_the_first_index(n):
+    """NaNs among a thread's chunks, in its first and in later groups of chunks, in the chunks behind the last whole group
+    and in the elements behind the last whole chunk; a row of NaN."""
+    g = torch.Generator("cpu").manual_seed(n)
+    x = randn(64, n, n)
+    for r in range(1, 63):
+        x[r, torch.randint(0, n, (1 + r % 5,), generator=g)] = float("nan")
+        x[r, int(torch.randint(0, n, (1,), generator=g))] = float("inf")
+    for r, first in ((8, n - 1), (9, n - 9), (10, n // 2), (11, 0)):
+        x[r] = 1.0
+        x[r, first:] = float("nan")
+    x[63] = float("nan")
+    got = greedy_sample(x)
+    assert torch.equal(got, ref(x))
+    assert got[8:12].tolist() == [n - 1, n - 9, n // 2, 0] and got[63] == 0
+
+
 def test_constant_and_minus_inf_rows():
     x = torch.full((4, 1000), float("-inf"), dtype=torch.bfloat16, device=DEV)
     x[1] = 0.0
