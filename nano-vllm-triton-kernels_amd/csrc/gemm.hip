@@ -381,9 +381,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_nt(const Mfm
       float gf[8], uf[8], o[8];
       unpack8(gv, gf);
       unpack8(uv, uf);
-      silu_bf16_n(gf, o);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] *= uf[e];
+      for (int e = 0; e < 8; ++e) o[e] = silu_bf16(gf[e]) * uf[e];
       const u32x4 v = pack8(o);
       uint16_t* d = g.c + int64_t(m) * g.scm + n;
       if (n + 8 <= n2 && (reinterpret_cast<uintptr_t>(d) & 15) == 0) {
