@@ -611,7 +611,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const Prefi
 // What bounded prefill_attention_kernel here: every K and V fragment that a wave of 32 queries reads from LDS feeds one
 // MFMA (128 bytes per clock and CU, the LDS rate), the K / V tiles pass through registers with per-key row arithmetic,
 // and the two waves of a SIMD run the softmax and the matrix products in phase, so they add up (a probe: an MFMA of 32
-// clocks leaves room for 4-5 other instructions of its SIMD, and 64 MFMAs and the ~450 others of a tile have to be
+// clocks leaves room for 4-5 other instructions of its SIMD, and 64 MFMAs and the ~310 others of a tile have to be
 // mixed to fit). Here
 //   - a fragment read from LDS feeds two MFMAs (64 queries per wave, one wave per SIMD: O and Q in 192 accumulation
 //     registers, two tiles' scores in 128 vector registers);
